@@ -6,18 +6,19 @@
 // O / l. head_dim is 128, as in the reference (:226).
 //
 // MI355X design:
-//  * Workgroup = one q head x (32 x waves) query rows, 32 rows per wave:
-//    8 waves (256 rows, one workgroup per compute unit) when the grid takes
-//    at least two rounds of those, else 128 rows: as two 4-wave halves that
-//    split the block's key tiles (even / odd) and merge in LDS, for grids of
-//    4+ blocks per head up to ~1.5 rounds, or as 4 waves (two per compute
-//    unit, heavy and light row blocks paired when the grid is resident in
-//    one round). Longest (last) row blocks first; the q heads of one kv head
-//    on one XCD so their K/V tiles share an L2.
-//  * Keys go in 64-key tiles. The K tile's E4M3 codes are copied unchanged
-//    into LDS by the LDS-DMA loads (global_load_lds_dwordx4, 16-byte chunks
-//    XOR-swizzled by row so the operand reads are bank-conflict free), ahead
-//    of use, with no registers or VALU work.
+//  * Rows: the q heads of one kv head are packed token by token (row r of a
+//    kv head: token r / G, head r % G), so a block of rows holds few tokens,
+//    its waves reach the diagonal in the same tile or the next, and the blocks
+//    of one kv head (on one XCD) share its K/V tiles in L2. 32 rows per wave;
+//    workgroups of 8 waves (256 rows, one per compute unit) or 4 (128 rows,
+//    two per compute unit). Longest (last) row blocks first.
+//  * Keys go in 64-key tiles, copied by LDS-DMA (global_load_lds) one and a
+//    half tiles or more ahead: K codes unchanged into a ring of three (16-byte
+//    chunks XOR-swizzled by row, so the operand reads are bank-conflict free),
+//    V codes into a ring of two that each wave copies and reads back for
+//    itself, scales into a ring of four. No load of the tile loop goes through
+//    registers, and the waits are explicit: the compiler would wait for every
+//    outstanding LDS-DMA before each LDS read.
 //  * Scores S^T = K Q^T run on the fp8 MFMA v_mfma_scale_f32_32x32x64_f8f6f4
 //    with A = the raw K codes from LDS and B = Q split into two E4M3
 //    parts: q * 2^a = hi + lo / 16 (a per row, so the row maximum lands in
@@ -35,19 +36,29 @@
 //  * V is dequantized into LDS as f16(code * v_scale), transposed to V^T in
 //    registers (v_perm) before the LDS write, and O^T += V^T P^T runs on
 //    v_mfma_f32_32x32x16_f16 with P^T straight from the score registers.
-//  * Buffers are separate LDS arrays indexed statically (the tile loop is
-//    unrolled), so the compiler sees the LDS-DMA into one buffer and the reads
-//    of another as independent. One barrier per tile, which waits only for
-//    the K copy the next tile needs.
-//  * 8-wave workgroups run two phase-shifted groups so that the softmax
-//    (VALU) of one wave meets the MFMAs of the other wave on its SIMD, and a
-//    wave in its softmax or P V runs at a higher issue priority than one in
-//    its score MFMAs; the 4-wave workgroups weave the next tile's copies and
-//    V staging between their own MFMAs.
+//  * The tile loop is software pipelined by half tiles (32 keys) and written
+//    in issue order (sched_barrier between the pieces): the P V MFMAs of one
+//    half alternate with the score MFMAs of the half a tile later (which are a
+//    dependent chain of four), and both run over the softmax of the half
+//    between them, the staging of the next V tile and the operand reads of the
+//    MFMAs ahead. Before, a wave did scores, softmax and P V one after the
+//    other, and the compiler put a wait for all outstanding copies in front of
+//    each tile's reads. What bounds it: one wave per SIMD (4-wave grids of up
+//    to one workgroup per compute unit) issues ~340 instructions per tile at
+//    one per ~5 cycles, 1.05 us a tile (1.6 before); two waves per SIMD run at
+//    57 % of the MFMA rate at ~1.9 GHz, where the part's power holds it (a
+//    large bf16 matrix product: 1.23 PFLOP/s; this kernel at 16384 tokens, 32
+//    heads 1.15). Measured, before -> now, us: 24 heads 1021 / 1500 / 1800
+//    tokens 27.2 -> 24.5, 34.8 -> 33.3, 43.3 -> 38.9; 28 heads 1700 48.4 ->
+//    37.5; 32 heads 2048 / 3000 / 4096 / 16384 55.4 -> 47.1, 97 -> 85.6, 139
+//    -> 136, 1913 -> 1905.
 //  * Key runs (flash_prefill_keysplit_launch, kPart): for chunks after a long
-//    cache, each (row block, q head) of the 4-wave kernel is split over
-//    gridDim.y workgroups, each walking one run of key tiles and storing
-//    partials in the split-K decode layout for the decode merge.
+//    cache, each row block of the 4-wave kernel is split over gridDim.y
+//    workgroups, each walking one run of key tiles and storing partials in the
+//    split-K decode layout for the decode merge.
+#include <climits>
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "launch.hpp"
 
@@ -74,37 +85,42 @@ __device__ __forceinline__ int vt_pos(int o) {
     return grp + 8 * h + 4 * a + (o & 3);
 }
 
-// Physical cache row of logical key `key` (identity unless paged: blocks of
-// 2^block_shift keys, logical block b at physical block block_table[b]).
-template <bool kPaged>
-__device__ __forceinline__ int pf_row(int key, const int* __restrict__ block_table,
-                                      int block_shift) {
-    if constexpr (kPaged) {
-        return (block_table[key >> block_shift] << block_shift) |
-               (key & ((1 << block_shift) - 1));
-    } else {
-        return key;
-    }
+// Row of q / out ([n_new, hq] rows of kHD) that row r of virtual head vhead's
+// packed rows holds: token r / pack, q head vhead * pack + r % pack.
+__device__ __forceinline__ int64_t packed_row(int r, int pack, int hq, int vhead) {
+    const int t = r / pack;
+    return static_cast<int64_t>(t) * hq + vhead * pack + (r - t * pack);
 }
 
-// Physical row of key `key` of the tile starting at key0, clamped to the last
-// key (a tile past the end maps to the last tile). Paged: the tile's two
-// 32-key halves each lie inside one block (blocks hold a power of two >= 32
-// keys), so two uniform lookups per tile suffice.
+// Where a tile's rows are: key0 (clamped to the last tile, so that a copy past
+// the end repeats it), the last row that exists, and, paged, the offsets
+// (physical - logical key) of its two 32-key halves, each of which lies in
+// one block (blocks hold a power of two >= 32 keys).
 template <bool kPaged>
 struct TileRows {
-    int key0, total, d_lo, d_hi;
-    __device__ __forceinline__ TileRows(int key0_, int total_, const int* __restrict__ bt,
+    int key0, rem, d_lo, d_hi;
+    __device__ __forceinline__ TileRows(int key0_, int total, const int* __restrict__ bt,
                                         int bshift)
-        : key0(min(key0_, (total_ - 1) & ~(kBN - 1))), total(total_), d_lo(0), d_hi(0) {
+        : key0(min(key0_, (total - 1) & ~(kBN - 1))), d_lo(0), d_hi(0) {
+        rem = total - 1 - key0;
         if constexpr (kPaged) {
-            d_lo = pf_row<true>(key0, bt, bshift) - key0;
-            d_hi = (key0 + 32 < total) ? pf_row<true>(key0 + 32, bt, bshift) - (key0 + 32) : d_lo;
+            d_lo = (bt[key0 >> bshift] << bshift) - (key0 & ~((1 << bshift) - 1));
+            d_hi = d_lo;
+            if (rem >= 32) {
+                const int k1 = key0 + 32;
+                d_hi         = (bt[k1 >> bshift] << bshift) - (k1 & ~((1 << bshift) - 1));
+            }
         }
     }
-    __device__ __forceinline__ int operator()(int i) const {   // i = key offset in the tile
-        const int key = min(key0 + i, total - 1);
-        return key + ((key - key0 < 32) ? d_lo : d_hi);
+    // Byte offset of the tile's row 0 as half `hi` counts its rows. Signed when
+    // paged: the second half's block can lie at physical row 0, so that its
+    // row 0 counted from the tile's start is row -32.
+    __device__ __forceinline__ int64_t base(bool hi, uint32_t stride) const {
+        if constexpr (kPaged) {
+            return static_cast<int64_t>(key0 + (hi ? d_hi : d_lo)) * static_cast<int64_t>(stride);
+        } else {
+            return static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(key0)) * stride);
+        }
     }
 };
 
@@ -113,54 +129,116 @@ __device__ __forceinline__ int k_chunk(int r, int c) {
     return r * kHD + 16 * (c ^ (r & 7));
 }
 
-// Issues the LDS-DMA copy of one K tile: slot s (16 bytes) holds chunk
-// (s & 7) ^ (row & 7) of row s >> 3, so that k_chunk() finds it.
-template <int kThreads, bool kPaged>
-__device__ __forceinline__ void k_tile_dma(uint8_t* dst, const uint8_t* __restrict__ k,
-                                           const TileRows<kPaged>& rows, int kvh, int hkv,
-                                           int tid) {
+// A lane's part of the tile copies, as byte offsets from the tile's first row
+// (32 bit; a row past the last key reads the last one: offsets grow with the
+// row, so the smaller of the two offsets is the clamped row's).
+template <int kWaves>
+struct TileLane {
+    uint32_t kstride, sstride;   // bytes per key: codes, scales
+    uint32_t krow, kcol;         // K copy: row offset of slot tid, its chunk
+    uint32_t vrow, vcol;         // V copy: row offset of its (even) key, its chunk
+    uint32_t srow;               // scale copy: offset of its key
+
+    // The wave's key pairs p (8 of 4 waves, 4 of 8): first key of pair p. Eight
+    // waves take the pairs whose V^T words are consecutive (vt_pos).
+    static __device__ __forceinline__ int pair_key(int wave, int p) {
+        return kWaves == 4 ? 16 * wave + 2 * p
+                           : 16 * (wave >> 1) + 4 * (wave & 1) + 2 * (p & 1) + 8 * (p >> 1);
+    }
+
+    __device__ __forceinline__ TileLane(int tid, int wave, int lane, int hkv) {
+        const int r = tid >> 3;
+        const int c = (tid & 7) ^ (r & 7);
+        kstride     = static_cast<uint32_t>(hkv) * kHD;
+        sstride     = static_cast<uint32_t>(hkv) * 4u;
+        krow        = static_cast<uint32_t>(r) * kstride;
+        kcol        = 16u * static_cast<uint32_t>(c);
+        // V rows of a wave in LDS: the even keys of its pairs, then the odd ones.
+        const int vr = lane >> 3;
+        const int vk = kWaves == 4 ? pair_key(wave, vr) : pair_key(wave, vr & 3) + (vr >> 2);
+        vrow         = static_cast<uint32_t>(vk) * kstride;
+        vcol         = 16u * static_cast<uint32_t>(lane & 7);
+        // Scales of a wave in LDS: v_scale of its keys pair by pair, then k_scale.
+        const int sk = lane & (kWaves == 4 ? 15 : 7);
+        srow         = static_cast<uint32_t>(pair_key(wave, sk >> 1) + (sk & 1)) * sstride;
+    }
+};
+
+// A pointer that every lane holds, in scalar registers.
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+    const uint64_t a  = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = static_cast<uint32_t>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(a))));
+    const uint32_t hi = static_cast<uint32_t>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(a >> 32))));
+    return reinterpret_cast<const uint8_t*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// One LDS-DMA of 16 (or 4) bytes per lane: lane l's bytes land at LDS address
+// to + 16 l (4 l). In assembly, because the compiler waits for every
+// outstanding LDS-DMA before any LDS read; the waits here are explicit.
+__device__ __forceinline__ void dma16(uint32_t to, const uint8_t* base, uint32_t off) {
+    base = uniform_ptr(base);
+    to   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(to)));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(to), "v"(off), "s"(base)
+                 : "memory");
+}
+// Lanes 0 .. kLanes - 1 only (the wave's lanes are all active).
+template <int kLanes>
+__device__ __forceinline__ void dma4_low(uint32_t to, const uint8_t* at) {
+    static_assert(kLanes == 16 || kLanes == 32, "");
+    to = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(to)));
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_hi, 0\n\ts_mov_b32 exec_lo, %2\n\t"
+                 "s_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1"
+                 :
+                 : "s"(to), "v"(at), "i"(kLanes == 32 ? -1 : 0xffff)
+                 : "memory");
+}
+
+// K tile: slot s (16 bytes) holds chunk (s & 7) ^ (row & 7) of row s >> 3, so
+// that k_chunk() finds it. kh: k + kvh rows. Slots of one copy lie in one
+// 32-row half.
+template <int kWaves, bool kPaged>
+__device__ __forceinline__ void k_tile_dma(uint32_t dst, const uint8_t* __restrict__ kh,
+                                           const TileRows<kPaged>& rows,
+                                           const TileLane<kWaves>& ln, int wave) {
+    const uint32_t lim = static_cast<uint32_t>(rows.rem) * ln.kstride;
 #pragma unroll
-    for (int rep = 0; rep < kKTile / 16 / kThreads; ++rep) {
-        const int      s   = tid + rep * kThreads;
-        const int      r   = s >> 3;
-        const int      c   = (s & 7) ^ (r & 7);
-        const uint8_t* src = k + (static_cast<int64_t>(rows(r)) * hkv + kvh) * kHD + 16 * c;
-        // The destination base is wave-uniform; lane l lands at base + 16 l.
-        __builtin_amdgcn_global_load_lds(src, dst + 16 * (s & ~(kWave - 1)), 16, 0, 0);
+    for (int rep = 0; rep < 8 / kWaves; ++rep) {
+        const bool hi = kWaves == 8 ? wave >= 4 : rep == 1;
+        dma16(dst + 1024u * static_cast<uint32_t>(wave + rep * kWaves),
+              kh + rows.base(hi, ln.kstride), min(ln.krow + rep * 32u * ln.kstride, lim) + ln.kcol);
     }
 }
 
-// Registers of the next tile's V staging: per unit, 8 E4M3 bytes (d0..d0+7)
-// of two consecutive keys and their v_scale; plus one k_scale.
-template <int kReps>
-struct VRaw {
-    u32x2 a[kReps], b[kReps];
-    float sa[kReps], sb[kReps];
-    float ks;
-};
-
-// V staging units: unit u = (key pair kp = u & 31, d group u >> 5 of 8 d).
-template <int kThreads, bool kPaged>
-__device__ __forceinline__ void v_tile_load(VRaw<4096 / 8 / kThreads>& r,
-                                            const uint8_t* __restrict__ v,
-                                            const float* __restrict__ ks,
-                                            const float* __restrict__ vs,
-                                            const TileRows<kPaged>& rows, int kvh, int hkv,
-                                            int tid) {
-    constexpr int kReps = 4096 / 8 / kThreads;
-#pragma unroll
-    for (int rep = 0; rep < kReps; ++rep) {
-        const int     u  = tid + rep * kThreads;
-        const int     kp = u & 31;
-        const int     d0 = 8 * (u >> 5);
-        const int64_t r0 = static_cast<int64_t>(rows(2 * kp)) * hkv + kvh;
-        const int64_t r1 = static_cast<int64_t>(rows(2 * kp + 1)) * hkv + kvh;
-        r.a[rep]  = *reinterpret_cast<const u32x2*>(v + r0 * kHD + d0);
-        r.b[rep]  = *reinterpret_cast<const u32x2*>(v + r1 * kHD + d0);
-        r.sa[rep] = vs[r0];
-        r.sb[rep] = vs[r1];
+// V tile: each wave copies its own 64 / kWaves keys (8 lanes per key), the
+// even keys of its pairs first, and later reads back only those.
+template <int kWaves, bool kPaged>
+__device__ __forceinline__ void v_tile_dma(uint32_t dst, const uint8_t* __restrict__ vh,
+                                           const TileRows<kPaged>& rows,
+                                           const TileLane<kWaves>& ln, int wave) {
+    const uint32_t lim  = static_cast<uint32_t>(rows.rem) * ln.kstride;
+    const uint8_t* base = vh + rows.base(wave >= kWaves / 2, ln.kstride);
+    const uint32_t to   = dst + static_cast<uint32_t>(wave * (kKTile / kWaves));
+    dma16(to, base, min(ln.vrow, lim) + ln.vcol);
+    if constexpr (kWaves == 4) {
+        dma16(to + 1024u, base, min(ln.vrow + ln.kstride, lim) + ln.vcol);
     }
-    r.ks = ks[static_cast<int64_t>(rows(tid & (kBN - 1))) * hkv + kvh];
+}
+
+// The scales of the wave's keys: v_scale, then k_scale.
+template <int kWaves, bool kPaged>
+__device__ __forceinline__ void scale_dma(uint32_t dst, const float* __restrict__ ksh,
+                                          const float* __restrict__ vsh,
+                                          const TileRows<kPaged>& rows,
+                                          const TileLane<kWaves>& ln, int wave, int lane) {
+    constexpr int  kKeys = 64 / kWaves;
+    const uint32_t lim   = static_cast<uint32_t>(rows.rem) * ln.sstride;
+    const int64_t  at    = rows.base(wave >= kWaves / 2, ln.sstride) + min(ln.srow, lim);
+    const uint8_t* base  = reinterpret_cast<const uint8_t*>(lane < kKeys ? vsh : ksh);
+    dma4_low<2 * kKeys>(dst + static_cast<uint32_t>(wave * 8 * kKeys), base + at);
 }
 
 // Exponent field of x alone: 2^floor(log2 x) for normal x > 0, 0 for 0.
@@ -168,47 +246,53 @@ __device__ __forceinline__ uint32_t pow2_bits(float x) {
     return __float_as_uint(x) & 0x7f800000u;
 }
 
-// Writes V'^T = f16(code * v_scale) for the staged units and the k_scale
-// factors of the tile. The two keys of a unit share the larger power of two
-// 2^e of their scales, applied exactly by the converter; the f16 factors
-// v_scale / 2^e (rounded once per key, a relative error below 2^-11 that
-// enters O linearly) are applied with one packed f16 multiply.
-template <int kThreads>
-__device__ __forceinline__ void v_tile_stage(const VRaw<4096 / 8 / kThreads>& r, uint16_t* vt,
-                                             float* kf, int tid, float scale_log2) {
-    constexpr int kReps = 4096 / 8 / kThreads;
-#pragma unroll
-    for (int rep = 0; rep < kReps; ++rep) {
-        const int      u   = tid + rep * kThreads;
-        const int      kp  = u & 31;
-        const int      d0  = 8 * (u >> 5);
-        const uint32_t e   = max(pow2_bits(r.sa[rep]), pow2_bits(r.sb[rep]));
-        const float    p   = __uint_as_float(e);
-        const float    inv = __uint_as_float(0x7f000000u - e);   // 2^-e
-        const f16x2    m   = {static_cast<_Float16>(r.sa[rep] * inv),
-                              static_cast<_Float16>(r.sb[rep] * inv)};
-        uint32_t*      col = reinterpret_cast<uint32_t*>(vt + vt_pos(2 * kp));
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const uint32_t wa = half ? r.a[rep].y : r.a[rep].x;
-            const uint32_t wb = half ? r.b[rep].y : r.b[rep].x;
-            // [a0 b0 a1 b1] and [a2 b2 a3 b3]: the two keys of one d per word.
-            const uint32_t lo = __builtin_amdgcn_perm(wb, wa, 0x05010400u);
-            const uint32_t hi = __builtin_amdgcn_perm(wb, wa, 0x07030602u);
-            const int      d  = d0 + 4 * half;
-            const f16x2 x0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, p, false) * m;
-            const f16x2 x1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, p, true) * m;
-            const f16x2 x2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, p, false) * m;
-            const f16x2 x3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, p, true) * m;
-            col[(d + 0) * (kVPitch / 2)] = __builtin_bit_cast(uint32_t, x0);
-            col[(d + 1) * (kVPitch / 2)] = __builtin_bit_cast(uint32_t, x1);
-            col[(d + 2) * (kVPitch / 2)] = __builtin_bit_cast(uint32_t, x2);
-            col[(d + 3) * (kVPitch / 2)] = __builtin_bit_cast(uint32_t, x3);
-        }
-    }
-    if (tid < kBN) {
-        kf[tid] = r.ks * scale_log2;
-    }
+// V'^T = f16(code * v_scale) of the staged units: the two keys of a unit share
+// the larger power of two 2^e of their scales, applied exactly by the
+// converter; the f16 factors v_scale / 2^e (rounded once per key, a relative
+// error below 2^-11 that enters O linearly) are applied with one packed f16
+// multiply.
+struct VFactor {
+    float p;   // 2^e
+    f16x2 m;
+};
+__device__ __forceinline__ VFactor v_factor(float sa, float sb) {
+    const uint32_t e   = max(pow2_bits(sa), pow2_bits(sb));
+    const float    inv = __uint_as_float(0x7f000000u - e);   // 2^-e
+    return {__uint_as_float(e),
+            f16x2{static_cast<_Float16>(sa * inv), static_cast<_Float16>(sb * inv)}};
+}
+
+// Word of V^T row d in LDS: rows of kVPitch f16 (conflict-free for the operand
+// reads, 32 consecutive rows), 16 words further per 32 rows, which spreads the
+// staging writes of lanes 16 d apart.
+__device__ __forceinline__ constexpr int vt_row(int d) {
+    return d * (kVPitch / 2) + 16 * (d >> 5);
+}
+constexpr int kVtWords = kHD * (kVPitch / 2) + 16 * (kHD / 32);
+
+// Stages four d of a key pair: wa, wb hold their codes of the two keys, col the
+// pair's V^T column at the first of them. swap: the lane writes d + 2, d + 3
+// first, so that lanes an odd multiple of 16 d apart use other banks.
+struct VOrder {
+    uint32_t sel0, sel1;   // byte selectors of the first and the second two d
+    int      at0, at1;     // their word offsets
+    __device__ __forceinline__ explicit VOrder(bool swap)
+        // [a0 b0 a1 b1] and [a2 b2 a3 b3]: the two keys of one d per word.
+        : sel0(swap ? 0x07030602u : 0x05010400u), sel1(swap ? 0x05010400u : 0x07030602u),
+          at0(swap ? kVPitch : 0), at1(swap ? 0 : kVPitch) {}
+};
+__device__ __forceinline__ void v_stage4(uint32_t wa, uint32_t wb, const VFactor& f,
+                                         const VOrder& v, uint32_t* col0, uint32_t* col1) {
+    const uint32_t w0 = __builtin_amdgcn_perm(wb, wa, v.sel0);
+    const uint32_t w1 = __builtin_amdgcn_perm(wb, wa, v.sel1);
+    const f16x2    x0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, f.p, false) * f.m;
+    const f16x2    x1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, f.p, true) * f.m;
+    const f16x2    x2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, f.p, false) * f.m;
+    const f16x2    x3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, f.p, true) * f.m;
+    col0[0]           = __builtin_bit_cast(uint32_t, x0);
+    col0[kVPitch / 2] = __builtin_bit_cast(uint32_t, x1);
+    col1[0]           = __builtin_bit_cast(uint32_t, x2);
+    col1[kVPitch / 2] = __builtin_bit_cast(uint32_t, x3);
 }
 
 // Four fp32 -> four E4M3 bytes (RNE; inputs within range).
@@ -232,57 +316,39 @@ constexpr int waitcnt_vm(int n) {
     return (n & 0xf) | (0x7 << 4) | (0xf << 8) | ((n >> 4) << 14);
 }
 
-// kEarly (4-wave workgroups, four or more row blocks per head): the first two
-// tiles' K copies and V loads go out before the q load, and q's eight loads
-// go out together, so the prologue waits for one memory round trip instead of
-// three. Smaller grids, the key split and the 8-wave kernel keep the order
-// below (measured slower there, or spilling).
+// Keeps the instruction scheduler from moving anything across: the tile loop
+// below is written in the order it is meant to issue.
+__device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
+
 // kPart (4-wave workgroups): the keys are split over gridDim.y workgroups per
-// (row block, q head); workgroup y takes the y-th run of
-// max(ceil(tiles / S), kPartMinTiles) key tiles and stores its rows'
-// partials (m in log2 units, l, unnormalized O) in the split-K decode layout
-// ([rows, S] m, [rows, S] l, [rows, S, D] O, rows t * Hq + h) for the decode
-// merge; a row with no key in the run stores m = -inf, l = 0 and, in a
-// workgroup that has keys, O = 0 (a workgroup without keys leaves O unwritten;
-// the merge drops slots with m = -inf). When run 0 holds every key (at most
-// kPartMinTiles tiles in all), it stores the normalized output instead and
-// the merge returns at once.
+// row block; workgroup y takes the y-th run of max(ceil(tiles / S),
+// kPartMinTiles) key tiles and stores its rows' partials (m in log2 units, l,
+// unnormalized O) in the split-K decode layout ([rows, S] m, [rows, S] l,
+// [rows, S, D] O, rows t * Hq + h) for the decode merge; a row with no key in
+// the run stores m = -inf, l = 0 and, in a workgroup that has keys, O = 0 (a
+// workgroup without keys leaves O unwritten; the merge drops slots with m =
+// -inf). When run 0 holds every key (at most kPartMinTiles tiles in all), it
+// stores the normalized output instead and the merge returns at once.
 constexpr int kPartMinTiles = 8;   // a run's minimum: short caches use few runs
-template <int kWaves, bool kPaged, bool kSplit = false, bool kEarly = false, bool kPart = false>
-__global__ __launch_bounds__(kWaves * kWave, kSplit ? 1 : 2) void flash_prefill_kernel(
+
+template <int kWaves, bool kPaged, bool kPart>
+__global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
     const uint8_t* __restrict__ k, const uint8_t* __restrict__ v,
     const float* __restrict__ ks, const float* __restrict__ vs, int n_new,
-    const int* __restrict__ cache_len, int hq, int hkv, float scale_log2,
-    const int* __restrict__ block_table, int block_shift, bool one_round,
+    const int* __restrict__ cache_len, int pack, int share, int hkv, float scale_log2,
+    const int* __restrict__ block_table, int block_shift, int first_wgs,
     float* __restrict__ partial, int num_splits) {
-    static_assert(!kSplit || kWaves == 8, "the key split pairs two 4-wave halves");
-    static_assert(!kEarly || (kWaves == 4 && !kSplit), "early issue: 4-wave workgroups only");
-    static_assert(!kPart || (kWaves == 4 && !kSplit && !kEarly), "key runs: 4-wave workgroups");
-    constexpr int kThreads = kWaves * kWave;
-    constexpr int kRowWaves = kSplit ? 4 : kWaves;  // waves with distinct rows
-    constexpr int kBM      = 32 * kRowWaves;        // query rows per workgroup
-    // Threads of one tile pipeline (the whole workgroup, or one split half).
-    constexpr int kPThreads = kSplit ? kThreads / 2 : kThreads;
-    constexpr int kReps    = 4096 / 8 / kPThreads;  // V staging units per thread
-    // Vector-memory operations of one v_tile_load (4 per unit, 1 k_scale).
-    constexpr int kWaitAllButVLoads = waitcnt_vm(4 * kReps + 1);
+    constexpr int kBM = 32 * kWaves;   // query rows per workgroup
+    // LDS-DMA operations of one tile: K and V 8 / kWaves each, scales 1.
+    constexpr int kCopies = 8 / kWaves;
+    constexpr int kOps    = 2 * kCopies + 1;
 
-    // Separate arrays per buffer (not one indexed array), so that the
-    // compiler sees the LDS-DMA into one K buffer and the operand reads from
-    // the other as independent and does not wait for the DMA before them.
-    __shared__ __attribute__((aligned(16))) uint8_t  sK0[kKTile];
-    __shared__ __attribute__((aligned(16))) uint8_t  sK1[kKTile];
-    __shared__ __attribute__((aligned(16))) uint8_t  sK2[kKTile];   // 8-wave path only
-    __shared__ __attribute__((aligned(16))) uint8_t  sK3[kKTile];   // 8-wave path only
-    __shared__ __attribute__((aligned(16))) uint16_t sVt0[kHD * kVPitch];
-    __shared__ __attribute__((aligned(16))) uint16_t sVt1[kHD * kVPitch];
-    __shared__ __attribute__((aligned(16))) float    sKf0[kBN];
-    __shared__ __attribute__((aligned(16))) float    sKf1[kBN];
-    __shared__ __attribute__((aligned(16))) uint16_t sVt2[kHD * kVPitch];   // not 4-wave
-    __shared__ __attribute__((aligned(16))) uint16_t sVt3[kHD * kVPitch];   // not 4-wave
-    __shared__ __attribute__((aligned(16))) float    sKf2[kBN];             // key split only
-    __shared__ __attribute__((aligned(16))) float    sKf3[kBN];             // key split only
+    __shared__ __attribute__((aligned(16))) uint8_t  sK[3 * kKTile];    // K codes: ring of three
+    __shared__ __attribute__((aligned(16))) uint8_t  sV[2 * kKTile];    // V codes: ring of two
+    __shared__ __attribute__((aligned(16))) uint32_t sVt[2 * kVtWords]; // V^T: ring of two
+    __shared__ __attribute__((aligned(16))) float    sKf[4 * kBN];      // k-factors: ring of four
+    __shared__ __attribute__((aligned(16))) float    sSc[4 * 128];      // scales: ring of four
 
     const int tid  = static_cast<int>(threadIdx.x);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -290,28 +356,28 @@ __global__ __launch_bounds__(kWaves * kWave, kSplit ? 1 : 2) void flash_prefill_
     const int qn   = lane & 31;   // query row of this lane within the wave
     const int h    = lane >> 5;   // k-group
 
-    // Heavy (last) row blocks first; q heads of one kv head on one XCD. When
-    // the whole grid is resident at once (one_round, two workgroups per
-    // compute unit), the second half of the grid runs the light blocks in
-    // ascending order, so the two workgroups sharing a compute unit pair a
-    // heavy block with a light one.
-    const int n_blk    = (n_new + kBM - 1) / kBM;
-    const int bid      = static_cast<int>(blockIdx.x);
-    const int half_wgs = (n_blk / 2) * hq;
-    const int blk      = (one_round && bid >= half_wgs) ? (bid - half_wgs) / hq
-                                                        : n_blk - 1 - bid / hq;
-    const int hb    = bid % hq;
-    const int qh    = ((hq & 7) == 0) ? ((hb & 7) * (hq >> 3) + (hb >> 3)) : hb;
-    const int kvh   = qh / (hq / hkv);
+    // Virtual head vhead: `pack` q heads of one kv head, whose rows are packed
+    // token by token (row r: token r / pack, head r % pack); each kv head has
+    // `share` of them. Heavy (last) row blocks first, the virtual heads of one
+    // kv head on one XCD.
+    const int n_rows  = n_new * pack;   // of one virtual head
+    const int n_heads = hkv * share;
+    const int n_blk   = (n_rows + kBM - 1) / kBM;
+    const int bid     = static_cast<int>(blockIdx.x);
+    const int blk     = bid >= first_wgs ? (bid - first_wgs) / n_heads : n_blk - 1 - bid / n_heads;
+    const int hb      = bid % n_heads;
+    const int vhead   = ((n_heads & 7) == 0) ? ((hb & 7) * (n_heads >> 3) + (hb >> 3)) : hb;
+    const int kvh     = vhead / share;
+    const int hq      = n_heads * pack;
 
     const int clen    = *cache_len;
     const int total   = clen + n_new;
     const int q0      = blk * kBM;
-    const int last    = min(q0 + kBM, n_new) - 1;
+    const int last    = (min(q0 + kBM, n_rows) - 1) / pack;   // the block's last token
     const int n_tiles = min((total + kBN - 1) / kBN, (clen + last) / kBN + 1);
     // kPart: this workgroup's run of key tiles [kt_lo, kt_hi).
-    [[maybe_unused]] int  kt_lo   = 0;
-    [[maybe_unused]] int  kt_hi   = 0;
+    int                   kt_lo   = 0;
+    int                   kt_hi   = n_tiles;
     [[maybe_unused]] bool one_run = false;   // kPart: run 0 holds every key
     if constexpr (kPart) {
         const int tiles_all = (total + kBN - 1) / kBN;
@@ -321,9 +387,9 @@ __global__ __launch_bounds__(kWaves * kWave, kSplit ? 1 : 2) void flash_prefill_
         kt_hi               = min(kt_lo + per, n_tiles);
         if (kt_hi <= kt_lo) {   // no key of this run for any row of the block: m, l only
             const int r = q0 + tid;
-            if (!one_run && tid < kBM && r < n_new) {
+            if (!one_run && tid < kBM && r < n_rows) {
                 const int64_t rows = static_cast<int64_t>(n_new) * hq;
-                const int64_t slot = (static_cast<int64_t>(r) * hq + qh) * num_splits +
+                const int64_t slot = packed_row(r, pack, hq, vhead) * num_splits +
                                      static_cast<int64_t>(blockIdx.y);
                 partial[slot]                     = -INFINITY;
                 partial[rows * num_splits + slot] = 0.0f;
@@ -332,56 +398,69 @@ __global__ __launch_bounds__(kWaves * kWave, kSplit ? 1 : 2) void flash_prefill_
         }
     }
 
-    // Key split: waves w and w + 4 hold the same rows; half g = w / 4 runs
-    // the key tiles kt = g, g + 2, g + 4, ... and the halves merge at the end.
-    const int split_g = kSplit ? (wave >> 2) : 0;
-    const int first_kt = kPart ? kt_lo : split_g;   // a wave's first tile
-    const int wq0     = q0 + (kSplit ? (wave & 3) : wave) * 32;   // first row of this wave
-    const int wlast   = min(wq0 + 31, n_new - 1);    // may be < wq0 (idle wave)
-    const int w_tiles = (wlast < wq0) ? 0 : (clen + wlast) / kBN + 1;
-    const int my_q    = wq0 + qn;
-    const int my_pos  = clen + my_q;
+    const int  wq0     = q0 + wave * 32;              // first row of this wave
+    const int  wlast   = min(wq0 + 31, n_rows - 1);   // may be < wq0 (idle wave)
+    const int  w_tiles = (wlast < wq0) ? 0 : (clen + wlast / pack) / kBN + 1;
+    // A half tile from a key past this one on crosses the diagonal of the wave's
+    // first row or the end of the keys.
+    const int  mask_from = min(clen + wq0 / pack - 31, total - 32);
+    const int  my_row  = wq0 + qn;                    // row of this lane
+    const bool has     = my_row < n_rows;
+    // The last key it sees, less 4 h (mask).
+    const int my_lim = min(clen + my_row / pack, total - 1) - 4 * h;
 
-    [[maybe_unused]] VRaw<kReps> pre_raw0, pre_raw1;
-    if constexpr (kEarly) {
-        const TileRows<kPaged> r0(0, total, block_table, block_shift);
-        const TileRows<kPaged> r1(kBN, total, block_table, block_shift);
-        k_tile_dma<kPThreads>(sK0, k, r0, kvh, hkv, tid);
-        v_tile_load<kPThreads>(pre_raw0, v, ks, vs, r0, kvh, hkv, tid);
-        k_tile_dma<kPThreads>(sK1, k, r1, kvh, hkv, tid);
-        v_tile_load<kPThreads>(pre_raw1, v, ks, vs, r1, kvh, hkv, tid);
+    const TileLane<kWaves> ln(tid, wave, lane, hkv);
+    const uint8_t* kh  = k + static_cast<int64_t>(kvh) * kHD;
+    const uint8_t* vh  = v + static_cast<int64_t>(kvh) * kHD;
+    const float*   ksh = ks + kvh;
+    const float*   vsh = vs + kvh;
+    const uint32_t sk_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sK));   // LDS addresses
+    const uint32_t sv_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sV));
+    const uint32_t ss_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sSc));
+    auto rows_of = [&](int kt) {
+        return TileRows<kPaged>(kt * kBN, total, block_table, block_shift);
+    };
+
+    // Prologue: the first tiles' copies and q all go out before anything
+    // waits. The copies of tiles 0 and 1 (and the scales of 2 and 3) first.
+    {
+        const TileRows<kPaged> r0 = rows_of(kt_lo), r1 = rows_of(kt_lo + 1);
+        const TileRows<kPaged> r2 = rows_of(kt_lo + 2), r3 = rows_of(kt_lo + 3);
+        scale_dma<kWaves, kPaged>(ss_at, ksh, vsh, r0, ln, wave, lane);
+        v_tile_dma<kWaves, kPaged>(sv_at, vh, r0, ln, wave);
+        k_tile_dma<kWaves, kPaged>(sk_at, kh, r0, ln, wave);
+        scale_dma<kWaves, kPaged>(ss_at + 512, ksh, vsh, r1, ln, wave, lane);
+        k_tile_dma<kWaves, kPaged>(sk_at + kKTile, kh, r1, ln, wave);
+        v_tile_dma<kWaves, kPaged>(sv_at + kKTile, vh, r1, ln, wave);
+        scale_dma<kWaves, kPaged>(ss_at + 1024, ksh, vsh, r2, ln, wave, lane);
+        scale_dma<kWaves, kPaged>(ss_at + 1536, ksh, vsh, r3, ln, wave, lane);
+        k_tile_dma<kWaves, kPaged>(sk_at + 2 * kKTile, kh, r2, ln, wave);
     }
-    // Q^T (B operand) as hi + lo E4M3 parts. Lane (row my_q, group h) holds,
+    // Q^T (B operand) as hi + lo E4M3 parts. Lane (row my_row, group h) holds,
     // for k-step j, d = 64j + 32h .. +32 (the same d the K operand lanes of
     // group h hold, so the MFMA pairs matching d).
     i32x8 qhi[2], qlo[2];
     int   sc_hi, sc_lo;
+    u32x4 qraw[2][4];
     {
-        const bool      has = my_q < n_new;
-        const uint16_t* qr  = q + (static_cast<int64_t>(has ? my_q : 0) * hq + qh) * kHD;
-        float           x[2][32];
-        float           amax = 0.0f;
-        [[maybe_unused]] u32x4 qraw[2][4];
-        if constexpr (kEarly) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    qraw[j][c] = *reinterpret_cast<const u32x4*>(qr + 64 * j + 32 * h + 8 * c);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        const uint16_t* qr = q + packed_row(has ? my_row : 0, pack, hq, vhead) * kHD;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                u32x4 w;
-                if constexpr (kEarly) {
-                    w = qraw[j][c];
-                } else {
-                    w = *reinterpret_cast<const u32x4*>(qr + 64 * j + 32 * h + 8 * c);
-                }
+                qraw[j][c] = *reinterpret_cast<const u32x4*>(qr + 64 * j + 32 * h + 8 * c);
+            }
+        }
+    }
+    pin();
+    {
+        float x[2][32];
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                u32x4 w = qraw[j][c];
                 if (!has) {
                     w = u32x4{0u, 0u, 0u, 0u};
                 }
@@ -434,580 +513,503 @@ __global__ __launch_bounds__(kWaves * kWave, kSplit ? 1 : 2) void flash_prefill_
     float m_ref = 0.0f;   // lazy reference maximum of this lane's row (log2 units)
     float l_run = 0.0f;
 
-    // S^T = K Q^T for one tile: per 32-key block, two k-steps of 64 d, each
-    // as hi and lo MFMAs sharing the K operand; all eight K operand reads are
-    // issued before the first MFMA.
-    auto qk = [&](const uint8_t* kbuf, f32x16 (&sc)[2]) {
-        i32x8 ka[2][2];
+    // V staging: this lane's key pair is pair lane / (4 kWaves / 2) of its wave,
+    // its d the kD following kD * (lane % (128 / kD)).
+    constexpr int   kD     = kWaves == 4 ? 16 : 8;
+    constexpr int   kParts = kD / 4;   // staged four d at a time
+    const int       vp     = lane / (kHD / kD);
+    const int       vd     = kD * (lane % (kHD / kD));
+    const VOrder    vorder((vd & 16) != 0);
+    uint32_t* const vcol   = sVt + vt_row(vd) + vt_pos(TileLane<kWaves>::pair_key(wave, vp)) / 2;
+    uint32_t* const vcol0  = vcol + vorder.at0;
+    uint32_t* const vcol1  = vcol + vorder.at1;
+    const uint8_t*  vraw   = sV + wave * (kKTile / kWaves) + vp * kHD + vd;
+    const float*    vsc    = sSc + wave * (128 / kWaves) + 2 * vp;
+    constexpr int   kKeys  = 64 / kWaves;
+    const int       kk     = lane & (kKeys - 1);
+    const float*    ksc    = sSc + wave * (128 / kWaves) + kKeys + kk;
+    float* const    kfw    = sKf + TileLane<kWaves>::pair_key(wave, kk >> 1) + (kk & 1);
+    struct VRaw {
+        uint32_t a[kParts], b[kParts];
+        f32x2    s;
+        float    ks;
+    };
+    // V codes and v_scales of tile i, k_scale of tile i + 1.
+    auto read_raw = [&](int i) {
+        using Codes      = std::conditional_t<kWaves == 4, u32x4, u32x2>;
+        const uint8_t* p = vraw + (i & 1) * kKTile;
+        const Codes    a = *reinterpret_cast<const Codes*>(p);
+        const Codes    b = *reinterpret_cast<const Codes*>(p + kKeys / 2 * kHD);
+        VRaw           r;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int r = 32 * kb + qn;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int   c0 = 4 * j + 2 * h;
-                const u32x4 lo = *reinterpret_cast<const u32x4*>(kbuf + k_chunk(r, c0));
-                const u32x4 hi = *reinterpret_cast<const u32x4*>(kbuf + k_chunk(r, c0 + 1));
-                ka[kb][j] = i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y),
-                                  static_cast<int>(lo.z), static_cast<int>(lo.w),
-                                  static_cast<int>(hi.x), static_cast<int>(hi.y),
-                                  static_cast<int>(hi.z), static_cast<int>(hi.w)};
-            }
+        for (int c = 0; c < kParts; ++c) {
+            r.a[c] = a[c];
+            r.b[c] = b[c];
         }
-        sc[0] = f32x16{};
-        sc[1] = f32x16{};
+        r.s  = *reinterpret_cast<const f32x2*>(vsc + (i & 3) * 128);
+        r.ks = ksc[((i + 1) & 3) * 128];
+        return r;
+    };
+    auto stage = [&](const VRaw& r, const VFactor& f, int i, int c) {   // d 4c .. 4c + 3
+        if (c < kParts) {
+            const int at = (i & 1) * kVtWords + 4 * c * (kVPitch / 2);
+            v_stage4(r.a[c], r.b[c], f, vorder, vcol0 + at, vcol1 + at);
+        }
+    };
+    auto stage_kf = [&](float k_scale, int i) { kfw[(i & 3) * kBN] = k_scale * scale_log2; };
+
+    // Tile 0's and 1's copies have landed; behind them are the scales of tiles
+    // 2 and 3 and K(2).
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 + kCopies));
+    pin();
+    {
+        const VRaw    r = read_raw(0);
+        const VFactor f = v_factor(r.s.x, r.s.y);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int c = 0; c < kParts; ++c) {
+            stage(r, f, 0, c);
+        }
+        stage_kf(ksc[0], 0);
+        stage_kf(r.ks, 1);
+    }
+    pin();
+    lds_barrier();
+    // V(2) over V(0), which this wave alone has read.
+    v_tile_dma<kWaves, kPaged>(sv_at, vh, rows_of(kt_lo + 2), ln, wave);
+    pin();
+
+    // ---- operand reads and pieces of a tile --------------------------------
+    // The K operand of one 32-key half: k-steps j = 0, 1.
+    const uint32_t k_at = k_chunk(qn, 2 * h);   // the other chunks: bits 4 and 6 flipped
+    auto read_k = [&](uint32_t at_ring, int half, int j, i32x8& ka) {
+        const uint8_t* b  = sK + half * 32 * kHD;
+        const uint32_t at = (at_ring + k_at) ^ (j ? 64u : 0u);
+        const u32x4    lo = *reinterpret_cast<const u32x4*>(b + at);
+        const u32x4    hi = *reinterpret_cast<const u32x4*>(b + (at ^ 16u));
+        ka = i32x8{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z),
+                   static_cast<int>(lo.w), static_cast<int>(hi.x), static_cast<int>(hi.y),
+                   static_cast<int>(hi.z), static_cast<int>(hi.w)};
+    };
+    // MFMA c (0..3) of a half's scores: k-step c / 2, hi then lo part of q.
+    auto qk = [&](const i32x8 (&ka)[2], f32x16& s, int c) {
+        const f32x16 z = c == 0 ? f32x16{} : s;
+        s = (c & 1) ? __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                          ka[c >> 1], qlo[c >> 1], z, 0, 0, 0, kE8M0One, 0, sc_lo)
+                    : __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                          ka[c >> 1], qhi[c >> 1], z, 0, 0, 0, kE8M0One, 0, sc_hi);
+        // Keeps the compiler from sinking the MFMA below a later branch.
+        asm volatile("" : "+v"(s));
+        pin();
+    };
+    auto read_kf = [&](int i, int half, f32x4 (&f)[4]) {
+        const float* b = sKf + (i & 3) * kBN + 32 * half + 4 * h;
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                sc[kb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                    ka[kb][j], qhi[j], sc[kb], 0, 0, 0, kE8M0One, 0, sc_hi);
-            }
+        for (int g = 0; g < 4; ++g) {
+            f[g] = *reinterpret_cast<const f32x4*>(b + 8 * g);
+        }
+    };
+    const uint32_t* const vrow = sVt + vt_row(qn) + 4 * h;
+    f16x8                 va[8];
+    // Operand of MFMA c (0..7) of a half's P V: d block c & 3, k-step c / 4.
+    auto read_v = [&](int i, int half, int c) {
+        const uint32_t* p = vrow + (i & 1) * kVtWords + (vt_row(32) * (c & 3)) + 8 * (2 * half + (c >> 2));
+        va[c] = __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(p));
+    };
+    auto scale4 = [&](f32x16& s, const f32x4 (&f)[4], int g) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                sc[kb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                    ka[kb][j], qlo[j], sc[kb], 0, 0, 0, kE8M0One, 0, sc_lo);
+        for (int e = 0; e < 4; ++e) {
+            s[4 * g + e] = fmaf(s[4 * g + e], f[g][e], -m_ref);
+        }
+    };
+    // Register r of a half is its key 8 (r / 4) + 4 h + r % 4; key0: the half's
+    // first key. Masks past the diagonal and past the last key.
+    auto mask = [&](f32x16& s, int key0) {
+        if (key0 > mask_from) {
+            const int lim = my_lim - key0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (8 * (r >> 2) + (r & 3) > lim) {
+                    s[r] = -INFINITY;
+                }
             }
         }
     };
-    // Softmax of tile kt's scores (in place) into the P^T operands:
-    // t = s * (k_scale * scale * log2 e) - m_ref (register r of block kb is key
-    // 32kb + 8(r/4) + 4h + r%4 of the tile), the causal / key-end mask only on
-    // tiles that cross the diagonal or the end of the keys (a wave-uniform
-    // branch), e = 2^t in fp32, p = e rounded to f16 for the P V MFMAs, and
-    // the row sum of the fp32 e (four partial sums of VALU adds, as the
-    // reference sums its fp32 exponentials; a v_dot2c sum of the f16 p runs on
-    // the MFMA pipe and measured ~1 % slower; the key-split kernel keeps that
-    // form for its register budget). Lazy reference maximum (exact): m_ref moves to the row
-    // maximum only on a wave's first tile or when a row sum exceeds 2^15 (some
-    // score more than 15 above m_ref); otherwise the tile needs no max
-    // reduction, no cross-lane step and no rescale of l and O. Every p and l
-    // use the same m_ref, and p <= 2^15 keeps every p inside the f16 range.
-    // The k-factors of the 32 keys a lane holds, read before the score MFMAs
-    // so that the LDS latency hides behind them.
-    auto load_kf = [&](const float* kfb, f32x4 (&kfv)[8]) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            kfv[i] = *reinterpret_cast<const f32x4*>(kfb + 32 * (i >> 2) + 8 * (i & 3) + 4 * h);
-        }
+    struct Sum {
+        float a, b;
     };
-    auto softmax = [&](f32x16 (&sx)[2], const f32x4 (&kfv)[8], int kt, f16x8 (&pop)[4]) {
-        __builtin_amdgcn_s_setprio(1);
-        const int key0 = kt * kBN;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-                const f32x4 f = kfv[4 * kb + rg];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    sx[kb][4 * rg + e] = fmaf(sx[kb][4 * rg + e], f[e], -m_ref);
-                }
-            }
-        }
-        if ((key0 + kBN - 1 > clen + wq0) || (key0 + kBN > total)) {
-            // Key kp is visible iff kp <= min(my_pos, total - 1): one compare
-            // of the tile offset (a constant per register) against a per-lane
-            // threshold.
-            const int lim = min(my_pos, total - 1) - key0 - 4 * h;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    if (32 * kb + 8 * (r >> 2) + (r & 3) > lim) {
-                        sx[kb][r] = -INFINITY;
-                    }
-                }
-            }
-        }
-        float psum  = 0.0f;
-        auto  exp_p = [&]() {
-            float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    f16x8 pw;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int   r  = 8 * half + 2 * i;
-                        const float e0 = __builtin_amdgcn_exp2f(sx[kb][r]);
-                        const float e1 = __builtin_amdgcn_exp2f(sx[kb][r + 1]);
-                        const f16x2 pp = {static_cast<_Float16>(e0), static_cast<_Float16>(e1)};
-                        if constexpr (kSplit) {
-                            // The key-split kernel sits at 256 VGPRs; the fp32
-                            // sum would spill there.
-                            part[i] = __builtin_amdgcn_fdot2(pp, f16x2{1.0f16, 1.0f16},
-                                                             part[i], false);
-                        } else {
-                            part[i] += e0 + e1;
-                        }
-                        pw[2 * i]     = pp.x;
-                        pw[2 * i + 1] = pp.y;
-                    }
-                    pop[2 * kb + half] = pw;
-                }
-            }
-            psum = (part[0] + part[1]) + (part[2] + part[3]);
-        };
-        exp_p();
-        if (__any((kt == first_kt) || !(psum <= 0x1p15f))) {
+    // Four of a half's exponentials: p into the P^T operands, the fp32 sums.
+    auto exp4 = [&](const f32x16& s, int g, f16x8 (&p)[2], Sum& sum) {
+        const float e0 = __builtin_amdgcn_exp2f(s[4 * g]);
+        const float e1 = __builtin_amdgcn_exp2f(s[4 * g + 1]);
+        const float e2 = __builtin_amdgcn_exp2f(s[4 * g + 2]);
+        const float e3 = __builtin_amdgcn_exp2f(s[4 * g + 3]);
+        sum.a = g == 0 ? e0 + e1 : sum.a + (e0 + e1);
+        sum.b = g == 0 ? e2 + e3 : sum.b + (e2 + e3);
+        p[g >> 1][4 * (g & 1) + 0] = static_cast<_Float16>(e0);
+        p[g >> 1][4 * (g & 1) + 1] = static_cast<_Float16>(e1);
+        p[g >> 1][4 * (g & 1) + 2] = static_cast<_Float16>(e2);
+        p[g >> 1][4 * (g & 1) + 3] = static_cast<_Float16>(e3);
+    };
+    // Lazy reference maximum (exact): m_ref moves to the row maximum of the
+    // half only on the run's first half tile or when a row's sum of a half
+    // exceeds 2^15 (some score more than 15 above m_ref); otherwise the half
+    // needs no max reduction, no cross-lane step and no rescale of l and O.
+    // Every p and l use the same m_ref, and p <= 2^15 keeps every p inside the
+    // f16 range.
+    auto settle = [&](f32x16& s, f16x8 (&p)[2], Sum& sum, bool first) {
+        if (__any(first || !(sum.a + sum.b <= 0x1p15f))) {
             float tmax = -INFINITY;
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    tmax = fmaxf(tmax, sx[kb][r]);
-                }
+            for (int r = 0; r < 16; ++r) {
+                tmax = fmaxf(tmax, s[r]);
             }
             tmax = wave_xor_max(tmax, 32);
             // The first tile sets the reference; later tiles only raise it. A
             // row that is here because another row of the wave overflowed may
             // sit far below its reference: lowering it would scale O and l by
             // 2^-tmax, which overflows.
-            const float delta = (kt == first_kt) ? ((tmax == -INFINITY) ? 0.0f : tmax)
-                                          : fmaxf(tmax, 0.0f);
-            const float alpha = (kt == first_kt) ? 1.0f : __builtin_amdgcn_exp2f(-delta);
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                sx[kb] -= delta;
-            }
+            const float delta = first ? ((tmax == -INFINITY) ? 0.0f : tmax) : fmaxf(tmax, 0.0f);
+            const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-delta);
+            s -= delta;
             m_ref += delta;
             l_run *= alpha;
 #pragma unroll
             for (int db = 0; db < 4; ++db) {
                 o[db] *= alpha;
             }
-            exp_p();
-        }
-        l_run += psum;
-        __builtin_amdgcn_s_setprio(0);
-    };
-    // O^T += V^T P^T, the operand reads running four MFMAs ahead.
-    // The softmax and the P V run at wave priority 1, the score MFMAs and
-    // the copies at 0: when both waves of a SIMD can issue, the one past its
-    // scores goes first (measured +3 % at 4K-16K; priority on the scores
-    // instead: -7 %).
-    auto pv = [&](const uint16_t* vtb, const f16x8 (&pop)[4]) {
-        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
-            const uint16_t* arow = vtb + (32 * db + qn) * kVPitch + 8 * h;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const f16x8 va = *reinterpret_cast<const f16x8*>(arow + 16 * t);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pop[t], o[db], 0, 0, 0);
+            for (int g = 0; g < 4; ++g) {
+                exp4(s, g, p, sum);
             }
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 2);
-#pragma unroll
-        for (int i = 0; i < 12; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 2);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 2);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 2);
-        __builtin_amdgcn_s_setprio(0);
+        l_run += sum.a + sum.b;
+    };
+    auto pv = [&](const f16x8 (&p)[2], int c) {   // MFMA c (0..7) of a half's P V
+        o[c & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[c], p[c >> 2], o[c & 3], 0, 0, 0);
+        pin();
     };
 
-    if constexpr (kWaves == 8 && !kSplit) {
-        // The two waves sharing a SIMD (w and w + 4) run each tile in
-        // different phase orders so that one's softmax (VALU) meets the
-        // other's MFMAs: the early group (waves 0-3) copies the next K tile
-        // and does scores, softmax, P V of tile kt; the late group (waves
-        // 4-7) does P V of tile kt - 1 (its P kept in registers across the
-        // barrier), scores and softmax of tile kt, then stages V(kt + 1) into
-        // the fourth V^T buffer of a ring of four.
-        const bool late = wave >= kWaves / 2;
-        const int  gtid = tid & (kThreads / 2 - 1);   // thread index within the group
-
-        constexpr int kGThreads = kThreads / 2;
-        constexpr int kGReps    = 4096 / 8 / kGThreads;
-        // K codes go through a ring of four buffers, copied two tiles ahead.
-        // Prologue: tile 0 staged by everyone, K(1) copied; V(1) into the
-        // late group's registers.
-        VRaw<kGReps> raw0, raw1;
-        {
-            const TileRows<kPaged> r0(0, total, block_table, block_shift);
-            const TileRows<kPaged> r1(kBN, total, block_table, block_shift);
-            k_tile_dma<kThreads>(sK0, k, r0, kvh, hkv, tid);
-            k_tile_dma<kThreads>(sK1, k, r1, kvh, hkv, tid);
-            VRaw<kReps> rz;
-            v_tile_load<kThreads>(rz, v, ks, vs, r0, kvh, hkv, tid);
-            v_tile_stage<kThreads>(rz, sVt0, sKf0, tid, scale_log2);
-            if (late) {
-                const TileRows<kPaged> r1(kBN, total, block_table, block_shift);
-                v_tile_load<kGThreads>(raw1, v, ks, vs, r1, kvh, hkv, gtid);
-            }
+    // Entering tile i, a wave holds P of its first half, the scores and the
+    // k-factors of its second, and the operands of the MFMAs ahead: V^T of the
+    // first half, K of the next tile's first half.
+    f32x16 sa, sb;
+    f16x8  pa[2], pb[2];
+    f32x4  kf[4];
+    Sum    sum;
+    i32x8  ka[2];
+    const int n_steps = kt_hi - kt_lo;
+    const int mine    = max(0, min(w_tiles - kt_lo, n_steps));
+    if (mine > 0) {
+        i32x8 kb[2];
+        read_k(0, 0, 0, ka[0]);
+        read_k(0, 0, 1, ka[1]);
+        read_k(0, 1, 0, kb[0]);
+        read_k(0, 1, 1, kb[1]);
+        read_kf(0, 0, kf);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            qk(ka, sa, c);
         }
-        __syncthreads();
-
-        auto kbuf4 = [&]<int R>() -> uint8_t* {
-            if constexpr (R == 0) return sK0;
-            else if constexpr (R == 1) return sK1;
-            else if constexpr (R == 2) return sK2;
-            else return sK3;
-        };
-        // V^T(kt) lives in buffer kt % 4: during tile kt the early group reads
-        // V^T(kt), the late group reads V^T(kt - 1) and then stages
-        // V^T(kt + 1), so the staging never writes a buffer that another
-        // wave of its group may still be reading.
-        auto vbuf4 = [&]<int R>() -> uint16_t* {
-            if constexpr (R == 0) return sVt0;
-            else if constexpr (R == 1) return sVt1;
-            else if constexpr (R == 2) return sVt2;
-            else return sVt3;
-        };
-        if (!late) {
-            constexpr int kDmaOps = kKTile / 16 / kGThreads;   // copies issued per tile
-            // Rows of the tile two ahead, looked up (paged) one tile before use.
-            TileRows<kPaged> rn(2 * kBN, total, block_table, block_shift);
-            auto tile = [&]<int R>(int kt) {
-                constexpr int  B    = R & 1;
-                const uint8_t* kcur = kbuf4.template operator()<R>();
-                uint8_t*       nk   = kbuf4.template operator()<(R + 2) & 3>();
-                const float*   kfb  = B ? sKf1 : sKf0;
-                const uint16_t* vtb = vbuf4.template operator()<R>();
-                const TileRows<kPaged> r2 = rn;
-                rn = TileRows<kPaged>((kt + 3) * kBN, total, block_table, block_shift);
-                k_tile_dma<kGThreads>(nk, k, r2, kvh, hkv, gtid);
-                if (kt < w_tiles) {
-                    f32x16 sx[2];
-                    f16x8  pop[4];
-                    f32x4  kfv[8];
-                    load_kf(kfb, kfv);
-                    qk(kcur, sx);
-                    softmax(sx, kfv, kt, pop);
-                    pv(vtb, pop);
-                }
-                // K(kt + 1), copied during the previous tile, must have landed;
-                // this tile's copy of K(kt + 2) stays in flight.
-                __builtin_amdgcn_s_waitcnt(waitcnt_vm(kDmaOps));
-                lds_barrier();
-            };
-            for (int kt = 0; kt < n_tiles; kt += 4) {
-                tile.template operator()<0>(kt);
-                if (kt + 1 < n_tiles) tile.template operator()<1>(kt + 1);
-                if (kt + 2 < n_tiles) tile.template operator()<2>(kt + 2);
-                if (kt + 3 < n_tiles) tile.template operator()<3>(kt + 3);
-            }
-        } else {
-            f16x8 pop_keep[4];
-            TileRows<kPaged> rn(2 * kBN, total, block_table, block_shift);
-            auto  tile = [&]<int R>(int kt) {
-                constexpr int  B     = R & 1;
-                const uint8_t* kcur  = kbuf4.template operator()<R>();
-                const float*   kfb   = B ? sKf1 : sKf0;
-                uint16_t*      vprev = vbuf4.template operator()<(R + 3) & 3>();   // V^T(kt - 1)
-                uint16_t*      vnext = vbuf4.template operator()<(R + 1) & 3>();   // V^T(kt + 1)
-                float*         nkf   = B ? sKf0 : sKf1;
-                VRaw<kGReps>&  rawc  = B ? raw1 : raw0;
-                VRaw<kGReps>&  rawn  = B ? raw0 : raw1;
-                const TileRows<kPaged> r2 = rn;
-                rn = TileRows<kPaged>((kt + 3) * kBN, total, block_table, block_shift);
-                if (kt >= 1 && kt - 1 < w_tiles) {
-                    pv(vprev, pop_keep);
-                }
-                v_tile_load<kGThreads>(rawc, v, ks, vs, r2, kvh, hkv, gtid);
-                if (kt < w_tiles) {
-                    f32x16 sx[2];
-                    f32x4  kfv[8];
-                    load_kf(kfb, kfv);
-                    qk(kcur, sx);
-                    softmax(sx, kfv, kt, pop_keep);
-                }
-                v_tile_stage<kGThreads>(rawn, vnext, nkf, gtid, scale_log2);
-                lds_barrier();
-            };
-            for (int kt = 0; kt < n_tiles; kt += 4) {
-                tile.template operator()<0>(kt);
-                if (kt + 1 < n_tiles) tile.template operator()<1>(kt + 1);
-                if (kt + 2 < n_tiles) tile.template operator()<2>(kt + 2);
-                if (kt + 3 < n_tiles) tile.template operator()<3>(kt + 3);
-            }
-            // P V of the last tile.
-            if (n_tiles - 1 < w_tiles) {
-                switch ((n_tiles - 1) & 3) {
-                    case 0: pv(sVt0, pop_keep); break;
-                    case 1: pv(sVt1, pop_keep); break;
-                    case 2: pv(sVt2, pop_keep); break;
-                    default: pv(sVt3, pop_keep); break;
-                }
-            }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            qk(kb, sb, c);
         }
-    } else {
-    // One tile pipeline per half G (the whole workgroup unless key split):
-    // the stream of tiles G, G + kStride, G + 2 kStride, ... Each half has its
-    // own LDS buffers; both halves take the same number of barriers.
-    constexpr int kStride = kSplit ? 2 : 1;
-    const int     ptid    = tid & (kPThreads - 1);   // thread index within the pipeline
-    auto pipeline = [&]<int G>() {
-    // V staging registers, two sets: raw0 holds the even tiles, raw1 the odd
-        // ones, so the loads of tile kt + 2 go out a whole tile before the
-        // staging of tile kt + 1 needs its registers.
-        // Prologue: the stream's first tile staged, the second's K copied
-        // and V in raw1. (Tile "kt + 1" below is the stream's next tile,
-        // kt + kStride.)
-        VRaw<kReps> raw0, raw1;
-        const int t0 = kPart ? kt_lo : G;   // the stream's first tile
-        {
-            const TileRows<kPaged> r0(t0 * kBN, total, block_table, block_shift);
-            const TileRows<kPaged> r1((t0 + kStride) * kBN, total, block_table, block_shift);
-            if constexpr (kEarly) {
-                raw0 = pre_raw0;
-                raw1 = pre_raw1;
-                v_tile_stage<kPThreads>(raw0, sVt0, sKf0, ptid, scale_log2);
-            } else {
-                k_tile_dma<kPThreads>(G ? sK2 : sK0, k, r0, kvh, hkv, ptid);
-                v_tile_load<kPThreads>(raw0, v, ks, vs, r0, kvh, hkv, ptid);
-                v_tile_stage<kPThreads>(raw0, G ? sVt2 : sVt0, G ? sKf2 : sKf0, ptid, scale_log2);
-                k_tile_dma<kPThreads>(G ? sK3 : sK1, k, r1, kvh, hkv, ptid);
-                v_tile_load<kPThreads>(raw1, v, ks, vs, r1, kvh, hkv, ptid);
-            }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            scale4(sa, kf, g);
         }
-        __syncthreads();
-
-        // Rows of the tiles one and two ahead, looked up (paged) a tile
-        // before use.
-        TileRows<kPaged> rn1((t0 + kStride) * kBN, total, block_table, block_shift);
-        TileRows<kPaged> rn2((t0 + 2 * kStride) * kBN, total, block_table, block_shift);
-        // One tile from buffer B (static, so each buffer is a distinct array).
-        auto tile = [&]<int B>(int kt) {
-            uint8_t*  kb0 = G ? sK2 : sK0;
-            uint8_t*  kb1 = G ? sK3 : sK1;
-            uint16_t* vb0 = G ? sVt2 : sVt0;
-            uint16_t* vb1 = G ? sVt3 : sVt1;
-            float*    fb0 = G ? sKf2 : sKf0;
-            float*    fb1 = G ? sKf3 : sKf1;
-            uint8_t*  kt_s = B ? kb1 : kb0;
-            uint16_t* vt   = B ? vb1 : vb0;
-            float*    kf   = B ? fb1 : fb0;
-            uint8_t*  nk   = B ? kb0 : kb1;
-            uint16_t* nvt  = B ? vb0 : vb1;
-            float*    nkf  = B ? fb0 : fb1;
-            // On entry V(kt + 1) is in registers rawn (loaded during tile
-            // kt - 1). This tile copies K(kt + 1) into K buffer 1 - B, loads
-            // V(kt + 2) into rawc (issued after the copy, so that waiting for
-            // all but the V loads at the barrier covers the copy) and stages
-            // V(kt + 1) into V^T buffer 1 - B. Past the end the copies repeat
-            // the last tile into idle buffers, which nobody reads; doing them
-            // unconditionally keeps the copies and the staging in the same
-            // scheduling regions as the MFMAs, whose execution hides their VALU
-            // work.
-            VRaw<kReps>& rawc = B ? raw1 : raw0;
-            VRaw<kReps>& rawn = B ? raw0 : raw1;
-            const TileRows<kPaged> r1 = rn1;
-            const TileRows<kPaged> r2 = rn2;
-            rn1 = rn2;
-            rn2 = TileRows<kPaged>((kt + 3 * kStride) * kBN, total, block_table, block_shift);
-            if (kt < w_tiles) {
-                k_tile_dma<kPThreads>(nk, k, r1, kvh, hkv, ptid);
-                v_tile_load<kPThreads>(rawc, v, ks, vs, r2, kvh, hkv, ptid);
-
-                // S^T = K Q^T: per 32-key block, two k-steps of 64 d, each as
-                // hi and lo MFMAs sharing the K operand.
-                f32x16 s[2];
+        mask(sa, kt_lo * kBN);
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) {
-                    s[kb] = f32x16{};
-                    const int r = 32 * kb + qn;
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int c0 = 4 * j + 2 * h;
-                        const u32x4 lo = *reinterpret_cast<const u32x4*>(kt_s + k_chunk(r, c0));
-                        const u32x4 hi = *reinterpret_cast<const u32x4*>(kt_s + k_chunk(r, c0 + 1));
-                        const i32x8 ka = {static_cast<int>(lo.x), static_cast<int>(lo.y),
-                                          static_cast<int>(lo.z), static_cast<int>(lo.w),
-                                          static_cast<int>(hi.x), static_cast<int>(hi.y),
-                                          static_cast<int>(hi.z), static_cast<int>(hi.w)};
-                        s[kb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            ka, qhi[j], s[kb], 0, 0, 0, kE8M0One, 0, sc_hi);
-                        s[kb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                            ka, qlo[j], s[kb], 0, 0, 0, kE8M0One, 0, sc_lo);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // VALU
-                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // global load
-                }
-
-                f16x8 pop[4];
-                f32x4 kfv[8];
-                load_kf(kf, kfv);
-                softmax(s, kfv, kt, pop);
-
-                // O^T += V^T P^T.
-#pragma unroll
-                for (int db = 0; db < 4; ++db) {
-                    const uint16_t* arow = vt + (32 * db + qn) * kVPitch + 8 * h;
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const f16x8 va = *reinterpret_cast<const f16x8*>(arow + 16 * t);
-                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pop[t], o[db], 0, 0, 0);
-                    }
-                }
-                v_tile_stage<kPThreads>(rawn, nvt, nkf, ptid, scale_log2);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);   // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);   // LDS read
-                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 1);   // VALU
-                    __builtin_amdgcn_sched_group_barrier(0x200, 1, 1);   // LDS write
-                }
-            } else {
-                k_tile_dma<kPThreads>(nk, k, r1, kvh, hkv, ptid);
-                v_tile_load<kPThreads>(rawc, v, ks, vs, r2, kvh, hkv, ptid);
-                v_tile_stage<kPThreads>(rawn, nvt, nkf, ptid, scale_log2);
-            }
-            // K(kt + 1) must have landed and the staged LDS writes be visible
-            // before the next tile; the V loads of tile kt + 2 stay in flight.
-            __builtin_amdgcn_s_waitcnt(kWaitAllButVLoads);
-            lds_barrier();
-        };
-
-        const int n_steps = kPart ? kt_hi - kt_lo : (n_tiles + kStride - 1) / kStride;
-        for (int i = 0; i < n_steps; i += 2) {
-            tile.template operator()<0>(t0 + kStride * i);
-            if (i + 1 < n_steps) {
-                tile.template operator()<1>(t0 + kStride * (i + 1));
-            }
+        for (int g = 0; g < 4; ++g) {
+            exp4(sa, g, pa, sum);
         }
-    };
-    if constexpr (kSplit) {
-        if (split_g == 0) {
-            pipeline.template operator()<0>();
-        } else {
-            pipeline.template operator()<1>();
-        }
-        // Merge of the halves: half 1 leaves O, m_ref and its lane's l in LDS
-        // (the tile buffers, free after the barrier), half 0 rescales both to
-        // the larger reference and stores. A half that saw no key of a row
-        // (row sum 0) has weight 0.
-        __syncthreads();
-        // The merge reuses the tile buffers: each V^T buffer holds one d block
-        // of O (16 floats per thread), sK0 holds m_ref and l of every thread.
-        static_assert(kHD * kVPitch * sizeof(uint16_t) >= 16 * kPThreads * sizeof(float),
-                      "a V^T buffer must hold a d block of O for every thread");
-        static_assert(kKTile >= 2 * kPThreads * sizeof(float),
-                      "a K buffer must hold m_ref and l for every thread");
-        float* mo[4] = {reinterpret_cast<float*>(sVt0), reinterpret_cast<float*>(sVt1),
-                        reinterpret_cast<float*>(sVt2), reinterpret_cast<float*>(sVt3)};
-        float* ml    = reinterpret_cast<float*>(sK0);   // [256] m_ref, [256] l
-        if (split_g == 1) {
-#pragma unroll
-            for (int db = 0; db < 4; ++db) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    mo[db][r * kPThreads + ptid] = o[db][r];
-                }
-            }
-            ml[ptid]             = m_ref;
-            ml[kPThreads + ptid] = l_run;
-        }
-        __syncthreads();
-        if (split_g == 1) {
-            return;
-        }
-        const float m1   = ml[ptid];
-        const float l1   = ml[kPThreads + ptid];
-        const bool  use1 = wave_xor_sum(l1, 32) > 0.0f;
-        const float mm   = use1 ? fmaxf(m_ref, m1) : m_ref;
-        const float f0   = __builtin_amdgcn_exp2f(m_ref - mm);
-        const float f1   = use1 ? __builtin_amdgcn_exp2f(m1 - mm) : 0.0f;
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o[db][r] = o[db][r] * f0 + mo[db][r * kPThreads + ptid] * f1;
-            }
-        }
-        l_run = l_run * f0 + l1 * f1;
-    } else {
-        pipeline.template operator()<0>();
+        settle(sa, pa, sum, true);
     }
+    // Rows of the tiles three and four ahead (paged: looked up a tile before use).
+    TileRows<kPaged> rn3 = rows_of(kt_lo + 3), rn4 = rows_of(kt_lo + 4);
+    uint32_t         ring = 0;   // byte offset of K(i) in its ring
+    // The copies of a tile: K(i + 3) over K(i), whose last reads a barrier has
+    // closed; V(i + 3) over V(i + 1), once this wave has read it; the scales
+    // of tile i + 4.
+    auto next_k = [&]() {
+        pin();
+        k_tile_dma<kWaves, kPaged>(sk_at + ring, kh, rn3, ln, wave);
+        pin();
+    };
+    auto next_v = [&](int i) {
+        pin();
+        v_tile_dma<kWaves, kPaged>(sv_at + ((i + 1) & 1) * kKTile, vh, rn3, ln, wave);
+        scale_dma<kWaves, kPaged>(ss_at + (i & 3) * 512, ksh, vsh, rn4, ln, wave, lane);
+        rn3 = rn4;
+        rn4 = rows_of(kt_lo + i + 5);
+        pin();
+    };
+    // The copies of the tile before must have landed and the staged LDS writes
+    // be visible; this tile's copies stay in flight.
+    auto tile_barrier = [&]() {
+        pin();
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(kOps));
+        lds_barrier();
+        pin();
+    };
+    auto ring_next = [](uint32_t r) {
+        return r == 2u * kKTile ? 0u : r + static_cast<uint32_t>(kKTile);
+    };
+    // K(0) is overwritten by the first tile's copy: its operand reads are done.
+    pin();
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kCopies));
+    lds_barrier();
+    pin();
+    // (In the order of the loop's reads, so that its waits count the same.)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        read_v(0, 0, c);
+        pin();
+        if (c == 3) {
+            read_k(kKTile, 0, 0, ka[0]);
+            pin();
+        }
+        if (c == 5) {
+            read_kf(0, 1, kf);
+            read_k(kKTile, 0, 1, ka[1]);
+            pin();
+        }
     }
 
+    // A tile that is not the workgroup's last.
+    auto tile = [&](int i) {
+        const uint32_t k1 = ring_next(ring);   // K(i + 1)
+        const uint32_t k2 = ring_next(k1);     // K(i + 2)
+        // P V of the first half and the next tile's first scores, under the
+        // softmax of the second half and the staging of V(i + 1); the operands
+        // of the part after this one are read as their registers come free.
+        pin();
+        scale4(sb, kf, 0);
+        scale4(sb, kf, 1);
+        pin();
+        if constexpr (kWaves == 8) {
+            __builtin_amdgcn_s_setprio(1);
+        }
+        pv(pa, 0);
+        read_v(i, 1, 0);
+        scale4(sb, kf, 2);
+        scale4(sb, kf, 3);
+        pin();
+        pv(pa, 1);
+        read_v(i, 1, 1);
+        const VRaw raw = read_raw(i + 1);
+        mask(sb, (kt_lo + i) * kBN + 32);
+        pin();
+        qk(ka, sa, 0);
+        exp4(sb, 0, pb, sum);
+        pin();
+        pv(pa, 2);
+        read_v(i, 1, 2);
+        pin();
+        pv(pa, 3);
+        read_v(i, 1, 3);
+        pin();
+        qk(ka, sa, 1);
+        read_k(k1, 1, 0, ka[0]);
+        exp4(sb, 1, pb, sum);
+        pin();
+        pv(pa, 4);
+        read_v(i, 1, 4);
+        const VFactor f = v_factor(raw.s.x, raw.s.y);
+        pin();
+        pv(pa, 5);
+        read_v(i, 1, 5);
+        exp4(sb, 2, pb, sum);
+        pin();
+        qk(ka, sa, 2);
+        exp4(sb, 3, pb, sum);
+        pin();
+        pv(pa, 6);
+        read_v(i, 1, 6);
+        pin();
+        pv(pa, 7);
+        read_v(i, 1, 7);
+        stage(raw, f, i + 1, 0);
+        pin();
+        qk(ka, sa, 3);
+        read_k(k1, 1, 1, ka[1]);
+        stage(raw, f, i + 1, 1);
+        pin();
+        if constexpr (kWaves == 8) {
+            __builtin_amdgcn_s_setprio(0);
+        }
+        settle(sb, pb, sum, false);
+        // P V of the second half and the next tile's second scores, under the
+        // softmax of the next tile's first half.
+        pin();
+        pv(pb, 0);
+        read_kf(i + 1, 0, kf);
+        stage(raw, f, i + 1, 2);
+        pin();
+        qk(ka, sb, 0);
+        stage(raw, f, i + 1, 3);
+        stage_kf(raw.ks, i + 2);
+        pin();
+        pv(pb, 1);
+        next_k();
+        scale4(sa, kf, 0);
+        scale4(sa, kf, 1);
+        pin();
+        pv(pb, 2);
+        scale4(sa, kf, 2);
+        scale4(sa, kf, 3);
+        pin();
+        mask(sa, (kt_lo + i + 1) * kBN);
+        pin();
+        qk(ka, sb, 1);
+        exp4(sa, 0, pa, sum);
+        pin();
+        pv(pb, 3);
+        next_v(i);
+        tile_barrier();
+        // V^T(i + 1) and K(i + 2) are there.
+        qk(ka, sb, 2);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            read_v(i + 1, 0, c);
+        }
+        read_k(k2, 0, 0, ka[0]);
+        exp4(sa, 1, pa, sum);
+        pin();
+        pv(pb, 4);
+        read_v(i + 1, 0, 4);
+        pin();
+        pv(pb, 5);
+        read_v(i + 1, 0, 5);
+        read_kf(i + 1, 1, kf);
+        exp4(sa, 2, pa, sum);
+        pin();
+        qk(ka, sb, 3);
+        read_k(k2, 0, 1, ka[1]);
+        exp4(sa, 3, pa, sum);
+        pin();
+        pv(pb, 6);
+        read_v(i + 1, 0, 6);
+        pin();
+        pv(pb, 7);
+        read_v(i + 1, 0, 7);
+        pin();
+        settle(sa, pa, sum, false);
+        ring = k1;
+    };
+    // Tiles with keys for this wave that are not the workgroup's last.
+    const int n_a = min(mine, n_steps - 1);
+    for (int i = 0; i < n_a; ++i) {
+        tile(i);
+    }
+    if (mine == n_steps) {   // the last tile
+        const int i = n_steps - 1;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            scale4(sb, kf, g);
+        }
+        mask(sb, (kt_lo + i) * kBN + 32);
+        pin();
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            pv(pa, c);
+            read_v(i, 1, c);
+            if (c & 1) {
+                exp4(sb, c >> 1, pb, sum);
+                pin();
+            }
+        }
+        settle(sb, pb, sum, false);
+        pin();
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            pv(pb, c);
+        }
+    } else {   // rows that see no further key: copy and stage for the other waves
+        for (int i = n_a; i < n_steps - 1; ++i) {
+            next_k();
+            const VRaw    raw = read_raw(i + 1);
+            const VFactor f   = v_factor(raw.s.x, raw.s.y);
+#pragma unroll
+            for (int c = 0; c < kParts; ++c) {
+                stage(raw, f, i + 1, c);
+            }
+            stage_kf(raw.ks, i + 2);
+            next_v(i);
+            tile_barrier();
+            ring = ring_next(ring);
+        }
+    }
+
+    // The copies past the last tile must have landed before the workgroup's LDS
+    // is given back.
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     const float l_tot = wave_xor_sum(l_run, 32);
+    // (The lane's row afresh, so that it takes no register over the loop.)
+    const int lane_e = static_cast<int>(
+        __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    const int he    = lane_e >> 5;
+    const int row_e = wq0 + (lane_e & 31);
+    if (row_e >= n_rows) {
+        return;
+    }
+    const int64_t row = packed_row(row_e, pack, hq, vhead);
     // kPart with a single live run (short caches): run 0 stores the output
     // itself, as the plain kernel does, and the merge skips the call.
     if (kPart && !one_run) {
-        if (my_q < n_new) {
-            const int64_t rows   = static_cast<int64_t>(n_new) * hq;
-            const int64_t slot   = (static_cast<int64_t>(my_q) * hq + qh) * num_splits +
-                                 static_cast<int64_t>(blockIdx.y);
-            const bool    any    = l_tot > 0.0f;
-            float*        part_o = partial + 2 * rows * num_splits + slot * kHD;
-            if (h == 0) {
-                partial[slot]                     = any ? m_ref : -INFINITY;
-                partial[rows * num_splits + slot] = l_tot;
-            }
-#pragma unroll
-            for (int db = 0; db < 4; ++db) {
-#pragma unroll
-                for (int rg = 0; rg < 4; ++rg) {
-                    *reinterpret_cast<f32x4*>(part_o + 32 * db + 8 * rg + 4 * h) =
-                        any ? f32x4{o[db][4 * rg], o[db][4 * rg + 1], o[db][4 * rg + 2],
-                                    o[db][4 * rg + 3]}
-                            : f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-            }
+        const int64_t rows   = static_cast<int64_t>(n_new) * hq;
+        const int64_t slot   = row * num_splits + static_cast<int64_t>(blockIdx.y);
+        const bool    any    = l_tot > 0.0f;
+        float*        part_o = partial + 2 * rows * num_splits + slot * kHD;
+        if (he == 0) {
+            partial[slot]                     = any ? m_ref : -INFINITY;
+            partial[rows * num_splits + slot] = l_tot;
         }
-        return;
-    }
-    if (my_q < n_new) {
-        const float inv_l = 1.0f / l_tot;
-        uint16_t*   orow  = out + (static_cast<int64_t>(my_q) * hq + qh) * kHD;
 #pragma unroll
         for (int db = 0; db < 4; ++db) {
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg) {
-                u32x2 w;
-                w.x = pack_bf16x2(o[db][4 * rg + 0] * inv_l, o[db][4 * rg + 1] * inv_l);
-                w.y = pack_bf16x2(o[db][4 * rg + 2] * inv_l, o[db][4 * rg + 3] * inv_l);
-                *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * rg + 4 * h) = w;
+                *reinterpret_cast<f32x4*>(part_o + 32 * db + 8 * rg + 4 * he) =
+                    any ? f32x4{o[db][4 * rg], o[db][4 * rg + 1], o[db][4 * rg + 2],
+                                o[db][4 * rg + 3]}
+                        : f32x4{0.f, 0.f, 0.f, 0.f};
             }
+        }
+        return;
+    }
+    const float inv_l = 1.0f / l_tot;
+    uint16_t*   orow  = out + row * kHD;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+            u32x2 w;
+            w.x = pack_bf16x2(o[db][4 * rg + 0] * inv_l, o[db][4 * rg + 1] * inv_l);
+            w.y = pack_bf16x2(o[db][4 * rg + 2] * inv_l, o[db][4 * rg + 3] * inv_l);
+            *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * rg + 4 * he) = w;
         }
     }
 }
 
-template <int kWaves, bool kSplit = false>
+template <int kWaves>
 void launch_prefill(uint16_t* out, const uint16_t* q, const uint8_t* k, const uint8_t* v,
                     const float* k_scale, const float* v_scale, int n_new, const int* cache_len,
-                    int hq, int hkv, float scale_log2, hipStream_t stream,
-                    const int* block_table, int block_shift, bool one_round) {
-    constexpr int kBM   = 32 * (kSplit ? 4 : kWaves);
-    const int     n_blk = (n_new + kBM - 1) / kBM;
-    const dim3    grid(static_cast<unsigned>(n_blk * hq));
-    // 4-wave grids of four or more row blocks per head: the early-issue
-    // prologue (+4-6 % at n = 2048-3072, 32 heads); grids of one to three
-    // blocks (n <= 384) keep the plain prologue (4-6 % faster there).
-    constexpr bool kEarlyOk = (kWaves == 4 && !kSplit);
-    const bool     early    = kEarlyOk && n_blk >= 4;
+                    int hq, int hkv, int pack, float scale_log2, hipStream_t stream,
+                    const int* block_table, int block_shift, int first_wgs) {
+    constexpr int kBM   = 32 * kWaves;
+    const int     share = hq / hkv / pack;
+    const int     n_blk = (n_new * pack + kBM - 1) / kBM;
+    const dim3    grid(static_cast<unsigned>(n_blk * hkv * share));
     if (block_table != nullptr) {
-        if (early) {
-            hipLaunchKernelGGL((flash_prefill_kernel<kWaves, true, kSplit, kEarlyOk>), grid,
-                               dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
-                               n_new, cache_len, hq, hkv, scale_log2, block_table, block_shift,
-                               one_round, nullptr, 1);
-        } else {
-            hipLaunchKernelGGL((flash_prefill_kernel<kWaves, true, kSplit>), grid,
-                               dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
-                               n_new, cache_len, hq, hkv, scale_log2, block_table, block_shift,
-                               one_round, nullptr, 1);
-        }
+        hipLaunchKernelGGL((flash_prefill_kernel<kWaves, true, false>), grid,
+                           dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
+                           n_new, cache_len, pack, share, hkv, scale_log2, block_table,
+                           block_shift, first_wgs, nullptr, 1);
     } else {
-        if (early) {
-            hipLaunchKernelGGL((flash_prefill_kernel<kWaves, false, kSplit, kEarlyOk>), grid,
-                               dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
-                               n_new, cache_len, hq, hkv, scale_log2, nullptr, 0, one_round,
-                               nullptr, 1);
-        } else {
-            hipLaunchKernelGGL((flash_prefill_kernel<kWaves, false, kSplit>), grid,
-                               dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
-                               n_new, cache_len, hq, hkv, scale_log2, nullptr, 0, one_round,
-                               nullptr, 1);
-        }
+        hipLaunchKernelGGL((flash_prefill_kernel<kWaves, false, false>), grid,
+                           dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
+                           n_new, cache_len, pack, share, hkv, scale_log2, nullptr, 0, first_wgs,
+                           nullptr, 1);
     }
 }
 
@@ -1020,11 +1022,12 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
                                int hq, int hkv, float scale_log2, hipStream_t stream,
                                const int* block_table, int block_shift) {
     constexpr int kBM   = 32 * 4;
-    const int     n_blk = (n_new + kBM - 1) / kBM;
-    const dim3    grid(static_cast<unsigned>(n_blk * hq), static_cast<unsigned>(num_splits));
-    hipLaunchKernelGGL((flash_prefill_kernel<4, kPaged, false, false, true>), grid,
+    const int     group = hq / hkv;
+    const int     n_blk = (n_new * group + kBM - 1) / kBM;
+    const dim3    grid(static_cast<unsigned>(n_blk * hkv), static_cast<unsigned>(num_splits));
+    hipLaunchKernelGGL((flash_prefill_kernel<4, kPaged, true>), grid,
                        dim3(4 * kWave), 0, stream, out, q, k, v, k_scale, v_scale, n_new,
-                       cache_len, hq, hkv, scale_log2, block_table, block_shift, false, partial,
+                       cache_len, group, 1, hkv, scale_log2, block_table, block_shift, INT_MAX, partial,
                        num_splits);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -1066,32 +1069,37 @@ hipError_t flash_prefill_launch(uint16_t* out, const uint16_t* q,
     if (head_dim != kHD) {
         return hipErrorInvalidValue;
     }
-    // 8-wave workgroups (256 rows, one per compute unit: half the staging
-    // per wave) when the grid takes at least two rounds of them. Below that,
-    // a compute unit holds too few waves to hide one tile's dependency chain
-    // (~1.4 us per 64-key tile for a lone wave): grids of up to 1.5 rounds of
-    // 128-row blocks, 4 blocks or more per head, split each block's keys over
-    // two 4-wave halves of one workgroup (heaviest block: half the serial
-    // tiles; 1500 x 24 heads 49 -> 36 us, 2048 x 24 50 us from 60); the rest
-    // take 4-wave workgroups (128 rows, two per compute unit) with heavy/light
-    // pairing, which balance the causal work of a single round better.
     int        cus = 0;
     hipError_t ce  = device_cu_count(&cus);
     if (ce != hipSuccess) {
         return ce;
     }
-    const float sl       = scale * kLog2e;
-    const int   n_blk128 = (n_new + 127) / 128;
-    if (((n_new + 255) / 256) * num_q_heads >= 2 * cus) {
+    const float sl    = scale * kLog2e;
+    const int   group = num_q_heads / num_kv_heads;
+    // The q heads of a kv head share blocks (packed rows) except in calls of up
+    // to 64 tokens, whose few blocks finish sooner one head each, spread over
+    // more compute units (17 x 32 heads 7.0 -> 6.4 us, 64 x 24 heads 8.2 -> 7.7).
+    const int pack   = n_new <= 64 ? 1 : group;
+    const int heads  = num_q_heads / pack;
+    const int rows   = n_new * pack;
+    const int wgs128 = (rows + 127) / 128 * heads;
+    // 8-wave workgroups (256 rows, one per compute unit, V staged once for all)
+    // when the grid takes 1.6 rounds of them or more; below that 4-wave
+    // workgroups (128 rows, two per compute unit), whose finer blocks balance
+    // the causal work better (8 / 4 waves, us: 24 heads 3600 tokens, 1.3
+    // rounds, 98.5 / 89.7; 32 heads 3000, 1.5 rounds, 85.5 / 85.5; 3600, 1.8
+    // rounds, 111.6 / 121.9; 4096, 2 rounds, 137 / 151).
+    if (5 * ((rows + 255) / 256) * heads >= 8 * cus) {
         launch_prefill<8>(out, q, k, v, k_scale, v_scale, n_new, cache_len, num_q_heads,
-                          num_kv_heads, sl, stream, block_table, block_shift, false);
-    } else if (n_blk128 >= 4 && 2 * n_blk128 * num_q_heads <= 3 * cus) {
-        launch_prefill<8, true>(out, q, k, v, k_scale, v_scale, n_new, cache_len, num_q_heads,
-                                num_kv_heads, sl, stream, block_table, block_shift, false);
+                          num_kv_heads, pack, sl, stream, block_table, block_shift, INT_MAX);
     } else {
-        const bool one_round = n_blk128 * num_q_heads <= 2 * cus;
+        // A grid that is resident in one round: one workgroup per compute unit,
+        // heaviest first, then the lightest blocks in ascending order, so that
+        // the workgroups that share a compute unit are a heavy and a light one.
+        const int per = cus / heads * heads;
         launch_prefill<4>(out, q, k, v, k_scale, v_scale, n_new, cache_len, num_q_heads,
-                          num_kv_heads, sl, stream, block_table, block_shift, one_round);
+                          num_kv_heads, pack, sl, stream, block_table, block_shift,
+                          per > 0 && wgs128 <= 2 * cus ? per : INT_MAX);
     }
     return hipGetLastError();
 }

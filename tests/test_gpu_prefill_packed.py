@@ -1,0 +1,59 @@
+"""The flash prefill's packed rows (the q heads of a kv head share row blocks)
+and its half-tile pipeline, at the sizes where they can go wrong: groups that
+do not divide a wave's 32 rows, blocks and waves that end mid-token, one to a
+few key tiles (the pipeline's first and last tile), the step from one head per
+block to packed heads (64 / 65 tokens), and the one-round ordering of the
+blocks on either side of one workgroup per compute unit. Against the oracle,
+with the attention tolerance of the other prefill tests."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+import runtherder_amd as R
+from gpu_util import DEV, NTHREADS, bf16_dev, bf16_host, f32_dev, int_dev, step, sync, u8_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def run(n, clen, hq, hkv, seed):
+    d, total = 128, clen + n
+    q = O.normal_bf16((n, hq, d), seed)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), seed + 1), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), seed + 2), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    step(f"packed prefill n={n} clen={clen} hq={hq} hkv={hkv}")
+    R.flash_prefill_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs), n,
+                         int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    got = bf16_host(out)
+    rows = min(n, 48)   # the last (longest) tokens in full, and the first ones
+    want = O.attention_f32(q[-rows:], k8, v8, ks, vs, rows, total - rows, hq, hkv, d, d ** -0.5,
+                           NTHREADS)
+    mx, mean = O.bf16_err(got[-rows:], want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+    first = min(n, 40)
+    want = O.attention_f32(q[:first], k8, v8, ks, vs, first, clen, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(got[:first], want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+    assert not np.isnan(got.astype(np.uint32) << 16).any()
+    return got
+
+
+# (tokens, cached, q heads, kv heads): G = 7, 3, 5, 1, 32
+@pytest.mark.parametrize("n,clen,hq,hkv", [
+    (1, 0, 28, 4), (2, 62, 28, 4), (19, 45, 24, 8), (64, 0, 15, 3), (65, 0, 15, 3),
+    (65, 127, 28, 4), (91, 37, 28, 4), (128, 64, 24, 8), (129, 63, 6, 6), (33, 300, 32, 1),
+    (86, 511, 24, 8)])
+def test_packed_rows_match_oracle(n, clen, hq, hkv):
+    run(n, clen, hq, hkv, 7000 + n)
+
+
+# Grids just below and above one 128-row workgroup per compute unit, and at the
+# end of the one-round ordering (two per compute unit): 8 kv heads, G = 1.
+@pytest.mark.parametrize("step_blocks", [-1, 0, 1])
+@pytest.mark.parametrize("rounds", [1, 2])
+def test_one_round_block_order(rounds, step_blocks):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = rounds * (cus // 8) + step_blocks
+    run(128 * blocks - 5, 0, 8, 8, 7300 + 10 * rounds + step_blocks)
