@@ -950,13 +950,13 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
         __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
     const int he    = lane_e >> 5;
     const int row_e = wq0 + (lane_e & 31);
-    if (row_e >= n_rows) {
-        return;
-    }
-    const int64_t row = packed_row(row_e, pack, hq, vhead);
     // kPart with a single live run (short caches): run 0 stores the output
     // itself, as the plain kernel does, and the merge skips the call.
     if (kPart && !one_run) {
+        if (row_e >= n_rows) {
+            return;
+        }
+        const int64_t row    = packed_row(row_e, pack, hq, vhead);
         const int64_t rows   = static_cast<int64_t>(n_new) * hq;
         const int64_t slot   = row * num_splits + static_cast<int64_t>(blockIdx.y);
         const bool    any    = l_tot > 0.0f;
@@ -977,16 +977,38 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
         }
         return;
     }
-    const float inv_l = 1.0f / l_tot;
-    uint16_t*   orow  = out + row * kHD;
+    // O / l in bf16 through LDS (every wave is past its last tile and every copy
+    // has landed), 64 d at a time, so that the stores are whole 128-byte runs
+    // of a row (16-byte pieces of 32 rows each before; per call, 32 heads: 128 /
+    // 300 / 4096 tokens 9.4 -> 8.6, 12.7 -> 11.9, 139.5 -> 136.5 us).
+    lds_barrier();
+    constexpr int kOPitch = 64 + 8;   // bf16 per row
+    static_assert(kWaves * 32 * kOPitch * 2 <= sizeof(sVt), "a wave's rows fit V^T's LDS");
+    uint16_t* const so    = reinterpret_cast<uint16_t*>(sVt) + wave * 32 * kOPitch;
+    const float     inv_l = 1.0f / l_tot;
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
+    for (int half = 0; half < 2; ++half) {
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-            u32x2 w;
-            w.x = pack_bf16x2(o[db][4 * rg + 0] * inv_l, o[db][4 * rg + 1] * inv_l);
-            w.y = pack_bf16x2(o[db][4 * rg + 2] * inv_l, o[db][4 * rg + 3] * inv_l);
-            *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * rg + 4 * he) = w;
+        for (int db = 0; db < 2; ++db) {
+            const f32x16& od = o[2 * half + db];
+#pragma unroll
+            for (int rg = 0; rg < 4; ++rg) {
+                u32x2 w;
+                w.x = pack_bf16x2(od[4 * rg + 0] * inv_l, od[4 * rg + 1] * inv_l);
+                w.y = pack_bf16x2(od[4 * rg + 2] * inv_l, od[4 * rg + 3] * inv_l);
+                *reinterpret_cast<u32x2*>(so + (lane_e & 31) * kOPitch + 32 * db + 8 * rg +
+                                          4 * he) = w;
+            }
+        }
+        // (One wave's LDS operations run in order.)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int   r = 8 * j + (lane_e >> 3);
+            const u32x4 w = *reinterpret_cast<const u32x4*>(so + r * kOPitch + 8 * (lane_e & 7));
+            if (wq0 + r < n_rows) {
+                *reinterpret_cast<u32x4*>(out + packed_row(wq0 + r, pack, hq, vhead) * kHD +
+                                          64 * half + 8 * (lane_e & 7)) = w;
+            }
         }
     }
 }
