@@ -5,12 +5,12 @@
 // the reference's fixed 32. Calls of 2 .. kPrefillSplitTokens tokens on shapes
 // the MFMA decode kernel serves run rth_attn_prefill_split over the same
 // scratch with num_splits / (2 n_new) splits (no reference counterpart: a few
-// tokens after a long cache as split-K decode; 16 / 64 tokens after 8K keys
-// 209 / 199 -> 18 / 34 us per call, at an empty cache up to ~2 us slower),
-// and at head_dim 128 calls of up to kPrefillRunsTokens tokens run it as the
-// flash prefill over key runs (128 / 256 tokens after 32K keys 828 / 830 ->
-// 98 / 187 us; at an empty cache 11 / 14 -> 19 / 27 us). For those the
-// scratch holds kPrefillRunTokenRuns token-runs (34 MB at 32 q heads).
+// tokens after a long cache as split-K decode; 16 tokens after 8K keys 209 ->
+// 17 us per call, at an empty cache up to ~2 us slower), and at head_dim 128
+// calls of up to kPrefillRunsTokens tokens run it as the flash prefill over
+// key runs (64 / 128 / 250 tokens after 32K keys 897 / 828 / 829 -> 51 / 83 /
+// 149 us; at an empty cache 2-6 us slower). For those the scratch holds
+// kPrefillRunTokenRuns token-runs (34 MB at 32 q heads).
 #pragma once
 
 #include <runtherder/attention/backend.h>
@@ -74,9 +74,11 @@ public:
 
     [[nodiscard]] int num_splits() const noexcept { return num_splits_; }
 
-    static constexpr int kPrefillSplitTokens  = 80;
-    static constexpr int kPrefillRunsTokens   = 256;
-    static constexpr int kPrefillRunTokenRuns = 2048;
+    // Above (head_dim 128): key runs, up to kPrefillSplitMostTokens where they fill the chip.
+    static constexpr int kPrefillSplitTokens     = 40;
+    static constexpr int kPrefillSplitMostTokens = 80;   // the decode route's most
+    static constexpr int kPrefillRunsTokens      = 256;
+    static constexpr int kPrefillRunTokenRuns    = 2048;
 
 private:
     // Split count of rth_attn_prefill_split for an n_new-token call, 0 when

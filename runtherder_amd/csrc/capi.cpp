@@ -152,8 +152,26 @@ int prefill_split_common(uint16_t* out, const uint16_t* q, const uint8_t* k, con
     }
     // Up to kPrefillSplitDecodeTokens tokens (or at head_dim != 128, which the
     // flash prefill does not serve): the decode split kernel over (token
-    // block, kv head) units; beyond, the flash prefill over key runs.
-    if (head_dim == 128 && n_new > rth::kPrefillSplitDecodeTokens) {
+    // block, kv head) units; beyond, the flash prefill over key runs. That
+    // also from kPrefillSplitRunTokens + 1 tokens where num_splits gives it a
+    // workgroup per compute unit: every block of tokens of the decode route
+    // reads the whole cache again (32 heads, decode route / 16 runs, us: 64
+    // tokens after 32K keys 86.6 / 51.1, 8K 31.0 / 26.5, 1K 15.6 / 17.6, none
+    // 9.5 / 11.0; 48 tokens 85.8 / 48.0, 30.4 / 25.6, 15.5 / 16.3, 9.0 / 10.7;
+    // 32 tokens 50.8 / 42, 22.0 / 23.6, 13.2 / 14.6, 7.9 / 10.1). With the few
+    // splits that suit the decode route (num_splits around CUs / n_new) it
+    // stays there.
+    bool runs = head_dim == 128 && n_new > rth::kPrefillSplitDecodeTokens;
+    if (head_dim == 128 && !runs && n_new > rth::kPrefillSplitRunTokens &&
+        rth::decode_mfma_supported(num_q_heads, num_kv_heads, head_dim)) {
+        int cus = 0;
+        if (int rc = check_hip(rth::device_cu_count(&cus), what)) {
+            return rc;
+        }
+        const long long rows = static_cast<long long>(n_new) * (num_q_heads / num_kv_heads);
+        runs = (rows + 127) / 128 * num_kv_heads * num_splits >= cus;
+    }
+    if (runs) {
         return check_hip(rth::flash_prefill_keysplit_launch(
                              out, q, k, v, k_scale, v_scale, partial, num_splits, n_new, cache_len,
                              num_q_heads, num_kv_heads, head_dim, scale, as_stream(stream),

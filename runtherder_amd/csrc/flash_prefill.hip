@@ -322,14 +322,13 @@ __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 
 // kPart (4-wave workgroups): the keys are split over gridDim.y workgroups per
 // row block; workgroup y takes the y-th run of max(ceil(tiles / S),
-// kPartMinTiles) key tiles and stores its rows' partials (m in log2 units, l,
+// run_min) key tiles and stores its rows' partials (m in log2 units, l,
 // unnormalized O) in the split-K decode layout ([rows, S] m, [rows, S] l,
 // [rows, S, D] O, rows t * Hq + h) for the decode merge; a row with no key in
 // the run stores m = -inf, l = 0 and, in a workgroup that has keys, O = 0 (a
 // workgroup without keys leaves O unwritten; the merge drops slots with m =
-// -inf). When run 0 holds every key (at most kPartMinTiles tiles in all), it
-// stores the normalized output instead and the merge returns at once.
-constexpr int kPartMinTiles = 8;   // a run's minimum: short caches use few runs
+// -inf). When run 0 holds every key (at most run_min tiles in all), it stores
+// the normalized output instead and the merge returns at once.
 
 template <int kWaves, bool kPaged, bool kPart>
 __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
@@ -338,7 +337,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
     const float* __restrict__ ks, const float* __restrict__ vs, int n_new,
     const int* __restrict__ cache_len, int pack, int share, int hkv, float scale_log2,
     const int* __restrict__ block_table, int block_shift, int first_wgs,
-    float* __restrict__ partial, int num_splits) {
+    float* __restrict__ partial, int num_splits, int run_min) {
     constexpr int kBM = 32 * kWaves;   // query rows per workgroup
     // LDS-DMA operations of one tile: K and V 8 / kWaves each, scales 1.
     constexpr int kCopies = 8 / kWaves;
@@ -381,7 +380,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
     [[maybe_unused]] bool one_run = false;   // kPart: run 0 holds every key
     if constexpr (kPart) {
         const int tiles_all = (total + kBN - 1) / kBN;
-        const int per       = max((tiles_all + num_splits - 1) / num_splits, kPartMinTiles);
+        const int per       = max((tiles_all + num_splits - 1) / num_splits, run_min);
         one_run             = tiles_all <= per;
         kt_lo               = static_cast<int>(blockIdx.y) * per;
         kt_hi               = min(kt_lo + per, n_tiles);
@@ -1026,12 +1025,12 @@ void launch_prefill(uint16_t* out, const uint16_t* q, const uint8_t* k, const ui
         hipLaunchKernelGGL((flash_prefill_kernel<kWaves, true, false>), grid,
                            dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
                            n_new, cache_len, pack, share, hkv, scale_log2, block_table,
-                           block_shift, first_wgs, nullptr, 1);
+                           block_shift, first_wgs, nullptr, 1, 1);
     } else {
         hipLaunchKernelGGL((flash_prefill_kernel<kWaves, false, false>), grid,
                            dim3(kWaves * kWave), 0, stream, out, q, k, v, k_scale, v_scale,
                            n_new, cache_len, pack, share, hkv, scale_log2, nullptr, 0, first_wgs,
-                           nullptr, 1);
+                           nullptr, 1, 1);
     }
 }
 
@@ -1043,20 +1042,26 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
                                float* partial, int num_splits, int n_new, const int* cache_len,
                                int hq, int hkv, float scale_log2, hipStream_t stream,
                                const int* block_table, int block_shift) {
-    constexpr int kBM   = 32 * 4;
+    // A run's minimum of tiles, so that short caches use few runs: what another
+    // run saves (1.05 us a tile) against the partials it writes for its rows
+    // and the merge reads (1K keys, 32 heads, minimum 2 / 4 / 8, us: 64 tokens
+    // 17.6 / 17.6 / 20.9; 128 tokens 26.1 / 22.6 / 25.1; 250 tokens 30.8 /
+    // 32.2 / 29.9).
+    const int     run_min = n_new <= 64 ? 2 : n_new <= 128 ? 4 : 8;
+    constexpr int kBM     = 32 * 4;
     const int     group = hq / hkv;
     const int     n_blk = (n_new * group + kBM - 1) / kBM;
     const dim3    grid(static_cast<unsigned>(n_blk * hkv), static_cast<unsigned>(num_splits));
     hipLaunchKernelGGL((flash_prefill_kernel<4, kPaged, true>), grid,
                        dim3(4 * kWave), 0, stream, out, q, k, v, k_scale, v_scale, n_new,
                        cache_len, group, 1, hkv, scale_log2, block_table, block_shift, INT_MAX, partial,
-                       num_splits);
+                       num_splits, run_min);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         return e;
     }
     return split_rows_merge_launch(out, partial, num_splits, cache_len, n_new * hq, n_new, kHD,
-                                   stream, kPartMinTiles);
+                                   stream, run_min);
 }
 
 }  // namespace

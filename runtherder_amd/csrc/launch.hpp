@@ -66,6 +66,7 @@ hipError_t flash_decode_launch(uint16_t* out, const uint16_t* q,
 // decode_scratch_floats(n_new * Hq, D, num_splits) floats.
 constexpr int kPrefillSplitMaxTokens       = 4096;   // rth_attn_prefill_split
 constexpr int kPrefillSplitDecodeTokens    = 80;     // above: the flash prefill over key runs
+constexpr int kPrefillSplitRunTokens       = 40;     // above, given splits that fill the chip: too
 constexpr int kPrefillSplitDecodeMaxTokens = 256;    // the decode kernel's route at D != 128
 hipError_t flash_prefill_split_launch(uint16_t* out, const uint16_t* q, const uint8_t* k,
                                      const uint8_t* v, const float* k_scale,
@@ -84,7 +85,7 @@ hipError_t split_rows_merge_launch(uint16_t* out, const float* partial, int num_
                                   hipStream_t stream, int run_min = 0);
 
 // The flash prefill (head_dim 128) with its keys split over num_splits
-// workgroups per (128-row block, q head), partials in the split-K decode
+// workgroups per 128-row block (tokens x q heads of a kv head), partials in the split-K decode
 // layout (decode_scratch_floats(n_new * Hq, 128, num_splits) floats), then
 // split_rows_merge_launch.
 hipError_t flash_prefill_keysplit_launch(uint16_t* out, const uint16_t* q, const uint8_t* k,

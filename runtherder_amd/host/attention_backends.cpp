@@ -43,20 +43,34 @@ AdaptiveAttention::AdaptiveAttention(const AttnConfig& config, int num_splits)
 }
 
 int AdaptiveAttention::prefill_split_count(int n_new) const noexcept {
-    if (n_new >= 2 && n_new <= kPrefillSplitTokens &&
-        rth_decode_path(config_.num_q_heads, config_.num_kv_heads, config_.head_dim) ==
-            RTH_DECODE_MFMA) {
-        return num_splits_ / (2 * n_new) > 1 ? num_splits_ / (2 * n_new) : 1;
+    if (n_new < 2 || n_new > kPrefillRunsTokens) {
+        return 0;
     }
-    if (n_new > kPrefillSplitTokens && n_new <= kPrefillRunsTokens && config_.head_dim == 128) {
-        // About two rounds of 4-wave workgroups, within the scratch.
-        const int blocks = (n_new + 127) / 128 * config_.num_q_heads;
+    const bool few = n_new <= kPrefillSplitMostTokens;
+    if (few && rth_decode_path(config_.num_q_heads, config_.num_kv_heads, config_.head_dim) !=
+                   RTH_DECODE_MFMA) {
+        return 0;
+    }
+    if (n_new > kPrefillSplitTokens && config_.head_dim == 128) {
+        // One to two rounds of the key runs' workgroups, within the scratch; past
+        // 16 runs only to fill the first.
+        const int rows   = n_new * (config_.num_q_heads / config_.num_kv_heads);
+        const int blocks = (rows + 127) / 128 * config_.num_kv_heads;
         int       runs   = 2 * cus_ / blocks;
-        runs             = runs < 16 ? runs : 16;
+        const int most   = (cus_ + blocks - 1) / blocks > 16 ? (cus_ + blocks - 1) / blocks : 16;
+        runs             = runs < most ? runs : most;
         runs             = runs < kPrefillRunTokenRuns / n_new ? runs : kPrefillRunTokenRuns / n_new;
-        return runs > 1 ? runs : 0;
+        if (!few) {
+            return runs > 1 ? runs : 0;
+        }
+        if (runs * blocks >= cus_) {
+            return runs;
+        }
     }
-    return 0;
+    if (!few) {
+        return 0;
+    }
+    return num_splits_ / (2 * n_new) > 1 ? num_splits_ / (2 * n_new) : 1;
 }
 
 void AdaptiveAttention::run(__hip_bfloat16* out, const __hip_bfloat16* q, const KVView& kv,

@@ -195,9 +195,10 @@ def flash_prefill_split_bf16(out, q, k, v, k_scale, v_scale, partial, num_splits
                              stream=None):
     """flash_prefill_bf16 split over the keys, for calls after a long cache
     (no reference counterpart; the reference walks every key serially per q
-    tile, flash_prefill.cu:34-241): up to 80 tokens as split-K decode over
-    (token block, kv head) units, beyond (head_dim 128) the flash prefill over
-    num_splits key runs per (row block, q head), both merged by the decode
+    tile, flash_prefill.cu:34-241): up to 80 tokens (40, where num_splits
+    fills the chip at head_dim 128) as split-K decode over (token block, kv
+    head) units, beyond (head_dim 128) the flash prefill over num_splits key
+    runs per block of 128 rows, both merged by the decode
     merge. partial: flash_split_scratch_floats(n_new * num_q_heads, head_dim,
     num_splits) floats; 1 <= n_new <= PREFILL_SPLIT_MAX_TOKENS."""
     _need(out, torch.bfloat16, "out"); _need(q, torch.bfloat16, "q")
@@ -443,7 +444,8 @@ class AttentionBackend:
         raise NotImplementedError
 
 
-PREFILL_SPLIT_TOKENS = 80
+PREFILL_SPLIT_TOKENS = 40        # above (head_dim 128): key runs where they fill the chip
+PREFILL_SPLIT_MOST_TOKENS = 80   # the decode route's most
 PREFILL_RUNS_TOKENS = 256
 PREFILL_RUN_TOKEN_RUNS = 2048
 
@@ -454,12 +456,12 @@ class AdaptiveAttention(AttentionBackend):
     device's (kv head, split) fill count. Calls of 2..PREFILL_SPLIT_TOKENS
     tokens on shapes the MFMA decode kernel serves take the split-K prefill
     (flash_prefill_split_bf16) over the same scratch, with num_splits //
-    (2 n_new) splits (no reference counterpart: per call, 16 / 64 tokens
-    after 8K keys 209 / 199 -> 18 / 34 us; at an empty cache up to ~2 us
-    slower); at head_dim 128, calls of up to PREFILL_RUNS_TOKENS tokens take
-    it as the flash prefill over key runs (128 / 256 tokens after 32K keys
-    828 / 830 -> 98 / 187 us; at an empty cache 11 / 14 -> 19 / 27 us), for
-    which the scratch holds PREFILL_RUN_TOKEN_RUNS token-runs."""
+    (2 n_new) splits (no reference counterpart: per call, 16 tokens after 8K
+    keys 209 -> 17 us; at an empty cache up to ~2 us slower); at head_dim 128,
+    calls of up to PREFILL_RUNS_TOKENS tokens take it as the flash prefill
+    over key runs (64 / 128 / 250 tokens after 32K keys 897 / 828 / 829 -> 51
+    / 83 / 149 us; at an empty cache 2-6 us slower), for which the scratch
+    holds PREFILL_RUN_TOKEN_RUNS token-runs."""
 
     def __init__(self, config: AttnConfig, num_splits: int | None = None, device="cuda"):
         self.config = config
@@ -473,15 +475,22 @@ class AdaptiveAttention(AttentionBackend):
 
     def _split_prefill_splits(self, n_new):
         c = self.config
-        if 2 <= n_new <= PREFILL_SPLIT_TOKENS:
-            if decode_path(c.num_q_heads, c.num_kv_heads, c.head_dim) != DECODE_MFMA:
-                return 0
-            return max(1, self.num_splits // (2 * n_new))
-        if PREFILL_SPLIT_TOKENS < n_new <= PREFILL_RUNS_TOKENS and c.head_dim == 128:
-            blocks = (n_new + 127) // 128 * c.num_q_heads
-            runs = min(2 * self.cus // blocks, 16, PREFILL_RUN_TOKEN_RUNS // n_new)
-            return runs if runs > 1 else 0
-        return 0
+        if not 2 <= n_new <= PREFILL_RUNS_TOKENS:
+            return 0
+        few = n_new <= PREFILL_SPLIT_MOST_TOKENS
+        if few and decode_path(c.num_q_heads, c.num_kv_heads, c.head_dim) != DECODE_MFMA:
+            return 0
+        if n_new > PREFILL_SPLIT_TOKENS and c.head_dim == 128:
+            # One to two rounds of the key runs' workgroups, within the scratch;
+            # past 16 runs only to fill the first.
+            blocks = (n_new * (c.num_q_heads // c.num_kv_heads) + 127) // 128 * c.num_kv_heads
+            runs = min(2 * self.cus // blocks, max(16, -(-self.cus // blocks)),
+                       PREFILL_RUN_TOKEN_RUNS // n_new)
+            if not few:
+                return runs if runs > 1 else 0
+            if runs * blocks >= self.cus:
+                return runs
+        return max(1, self.num_splits // (2 * n_new)) if few else 0
 
     def run(self, out, q, kv, n_new, cache_len, stream=None):
         c = self.config

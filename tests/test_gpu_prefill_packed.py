@@ -57,3 +57,37 @@ def test_one_round_block_order(rounds, step_blocks):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     blocks = rounds * (cus // 8) + step_blocks
     run(128 * blocks - 5, 0, 8, 8, 7300 + 10 * rounds + step_blocks)
+
+
+# Key runs of few tokens (41..80 with splits that fill the chip): run minimum
+# of 2 / 4 tiles on both sides of one run, ragged last runs, runs without keys
+# for the first rows, G = 3, 4, 7, and the split count just below the switch.
+@pytest.mark.parametrize("n,clen,hq,hkv,splits", [
+    (41, 0, 24, 8, 32), (48, 80, 32, 8, 16), (48, 81, 32, 8, 16), (64, 64, 32, 8, 16),
+    (64, 65, 32, 8, 16), (65, 191, 32, 8, 16), (66, 191, 32, 8, 16), (80, 1000, 28, 4, 22),
+    (80, 3001, 24, 8, 15), (50, 5000, 28, 4, 64), (64, 3000, 32, 8, 15)])
+def test_few_token_key_runs_match_oracle(n, clen, hq, hkv, splits):
+    d, total = 128, clen + n
+    q = O.normal_bf16((n, hq, d), 7500 + n)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7501 + n), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7502 + n), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    step(f"key runs n={n} clen={clen} hq={hq} hkv={hkv} splits={splits}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    want = O.attention_f32(q, k8, v8, ks, vs, n, clen, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(bf16_host(out), want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+
+
+def test_few_token_key_runs_refuse_what_the_decode_route_refused():
+    hq, hkv, d = 17, 1, 128   # a group the MFMA decode kernel does not serve
+    out = torch.empty((64, hq, d), dtype=torch.bfloat16, device=DEV)
+    kv = torch.zeros((100, hkv, d), dtype=torch.uint8, device=DEV)
+    s = torch.zeros((100, hkv), dtype=torch.float32, device=DEV)
+    part = R.new_flash_split_scratch(64 * hq, d, 128)
+    with pytest.raises(R._ffi.RthError, match="head_dim"):
+        R.flash_prefill_split_bf16(out, out, kv, kv, s, s, part, 128, 64, int_dev(0), hq, hkv, d,
+                                   0.1)
