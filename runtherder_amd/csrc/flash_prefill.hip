@@ -55,7 +55,8 @@
 //  * Key runs (flash_prefill_keysplit_launch, kPart): for chunks after a long
 //    cache, each row block of the 4-wave kernel is split over gridDim.y
 //    workgroups, each walking one run of key tiles and storing partials in the
-//    split-K decode layout for the decode merge.
+//    split-K decode layout for a merge of its own.
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -324,7 +325,7 @@ __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 // row block; workgroup y takes the y-th run of max(ceil(tiles / S),
 // run_min) key tiles and stores its rows' partials (m in log2 units, l,
 // unnormalized O) in the split-K decode layout ([rows, S] m, [rows, S] l,
-// [rows, S, D] O, rows t * Hq + h) for the decode merge; a row with no key in
+// [rows, S, D] O, rows t * Hq + h) for the merge; a row with no key in
 // the run stores m = -inf, l = 0 and, in a workgroup that has keys, O = 0 (a
 // workgroup without keys leaves O unwritten; the merge drops slots with m =
 // -inf). When run 0 holds every key (at most run_min tiles in all), it stores
@@ -1012,6 +1013,93 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
     }
 }
 
+// Merges the key runs' partials: out = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s -
+// M) l_s over the live runs (derived as the prefill kernel does). kSub groups
+// of 32 lanes per row (16 bytes of each O_s per lane; group i takes runs i, i +
+// kSub, ...). Many rows (few runs each) are bound by the partials' bytes, 520
+// per row and run, few rows by the loads' round trips; only the live runs are
+// read. Per call at 32 q heads / 8 kv heads, 64 / 160 / 250 tokens, with the
+// decode's whole-row merge (a workgroup of 128 per row, 32 slots read whatever
+// the count) -> with this one: empty cache 10.3 / 15.1 / 18.7 -> 9.0 / 11.1 /
+// 12.4 us, 1K keys 17.6 / 26.0 / 30.0 -> 13.6 / 22.9 / 26.0, 8K keys 26.5 /
+// 40.5 / 53.8 -> 23.5 / 41.0 / 51.6.
+constexpr int kMergeThreads = 256;
+template <int kSub>
+__global__ __launch_bounds__(kMergeThreads) void flash_prefill_merge_kernel(
+    uint16_t* __restrict__ out, const float* __restrict__ partial, int num_splits,
+    const int* __restrict__ cache_len, int rows, int n_new, int run_min) {
+    constexpr int kRows = kMergeThreads / (32 * kSub);
+    static_assert(kSub == 1 || kSub == 2, "a row's lanes lie in one wave");
+    const int tiles = (*cache_len + n_new + kBN - 1) / kBN;
+    const int per   = max((tiles + num_splits - 1) / num_splits, run_min);
+    const int live  = (tiles + per - 1) / per;
+    if (live == 1) {   // run 0 stored the output itself
+        return;
+    }
+    const int     hl  = static_cast<int>(threadIdx.x) & 31;
+    const int     sub = static_cast<int>(threadIdx.x) / 32 % kSub;
+    const int64_t hs  = static_cast<int64_t>(rows) * num_splits;
+    for (int row = static_cast<int>(blockIdx.x) * kRows +
+                   static_cast<int>(threadIdx.x) / (32 * kSub);
+         row < rows; row += static_cast<int>(gridDim.x) * kRows) {
+        const int64_t slot0 = static_cast<int64_t>(row) * num_splits;
+        const float*  pm    = partial + slot0;
+        const float*  pl    = partial + hs + slot0;
+        const float*  po    = partial + 2 * hs + slot0 * kHD + 4 * hl;
+        float         m[8], ls[8];
+        f32x4         os[8];
+        auto load8 = [&](int s0) {   // runs s0 + u kSub, clamped to the live ones
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = min(s0 + u * kSub, live - 1);
+                m[u]        = pm[i];
+                ls[u]       = pl[i];
+                os[u]       = *reinterpret_cast<const f32x4*>(po + static_cast<int64_t>(i) * kHD);
+            }
+        };
+        float big = pm[min(hl, live - 1)];   // M
+        load8(sub);
+        for (int i = hl + 32; i < live; i += 32) {
+            big = fmaxf(big, pm[i]);
+        }
+#pragma unroll
+        for (int x = 1; x < 32; x <<= 1) {
+            big = fmaxf(big, __shfl_xor(big, x, 32));
+        }
+        float l   = 0.0f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = sub;;) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                // A run without keys of the row (m = -inf) may hold no O at all.
+                const bool  use = s0 + u * kSub < live && m[u] != -INFINITY;
+                const float f   = use ? __builtin_amdgcn_exp2f(m[u] - big) : 0.0f;
+                acc += (use ? os[u] : f32x4{0.f, 0.f, 0.f, 0.f}) * f;
+                l += (use ? ls[u] : 0.0f) * f;
+            }
+            s0 += 8 * kSub;
+            if (s0 >= live) {
+                break;
+            }
+            load8(s0);
+        }
+        if constexpr (kSub == 2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[e] += __shfl_xor(acc[e], 32);
+            }
+            l += __shfl_xor(l, 32);
+        }
+        if (sub == 0) {
+            const float inv = __builtin_amdgcn_rcpf(l);   // 1 ulp; the output is bf16
+            u32x2       w;
+            w.x = pack_bf16x2(acc[0] * inv, acc[1] * inv);
+            w.y = pack_bf16x2(acc[2] * inv, acc[3] * inv);
+            *reinterpret_cast<u32x2*>(out + static_cast<int64_t>(row) * kHD + 4 * hl) = w;
+        }
+    }
+}
+
 template <int kWaves>
 void launch_prefill(uint16_t* out, const uint16_t* q, const uint8_t* k, const uint8_t* v,
                     const float* k_scale, const float* v_scale, int n_new, const int* cache_len,
@@ -1034,8 +1122,8 @@ void launch_prefill(uint16_t* out, const uint16_t* q, const uint8_t* k, const ui
     }
 }
 
-// The flash prefill with its keys split over num_splits workgroups per (row
-// block, q head), then the decode merge over the n_new * Hq rows.
+// The flash prefill with its keys split over num_splits workgroups per row
+// block, then the merge of the n_new * Hq rows.
 template <bool kPaged>
 hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* k,
                                const uint8_t* v, const float* k_scale, const float* v_scale,
@@ -1060,8 +1148,17 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
     if (e != hipSuccess) {
         return e;
     }
-    return split_rows_merge_launch(out, partial, num_splits, cache_len, n_new * hq, n_new, kHD,
-                                   stream, run_min);
+    const int rows = n_new * hq;
+    // At most eight workgroups per compute unit (256), 32 waves: all resident. A
+    // whole wave per row up to 4096 rows; the line at 8192 instead, 160 / 200
+    // tokens x 32 heads: empty cache 11.0 / 11.3 -> 11.3 / 11.6 us, 8K keys 41.4 /
+    // 47.2 -> 40.6 / 47.9, 32K 100.4 / 123.8 -> 101.6 / 126.3.
+    const bool wide = rows <= 4096;
+    const int  wgs  = std::min((rows * (wide ? 64 : 32) + kMergeThreads - 1) / kMergeThreads, 2048);
+    hipLaunchKernelGGL(wide ? flash_prefill_merge_kernel<2> : flash_prefill_merge_kernel<1>,
+                       dim3(static_cast<unsigned>(wgs)), dim3(kMergeThreads), 0, stream, out,
+                       partial, num_splits, cache_len, rows, n_new, run_min);
+    return hipGetLastError();
 }
 
 }  // namespace

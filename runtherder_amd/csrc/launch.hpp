@@ -76,18 +76,10 @@ hipError_t flash_prefill_split_launch(uint16_t* out, const uint16_t* q, const ui
                                      hipStream_t stream, const int* block_table = nullptr,
                                      int block_shift = 0);
 
-// The decode merge over `rows` rows of num_splits partials each (whole-row
-// workgroups): out row r = the merged row r; the live slots follow from
-// *cache_len + n_tok keys as in the split kernels, or (run_min > 0) as the
-// flash prefill's key runs of max(ceil(tiles / S), run_min) 64-key tiles.
-hipError_t split_rows_merge_launch(uint16_t* out, const float* partial, int num_splits,
-                                  const int* cache_len, int rows, int n_tok, int head_dim,
-                                  hipStream_t stream, int run_min = 0);
-
 // The flash prefill (head_dim 128) with its keys split over num_splits
 // workgroups per 128-row block (tokens x q heads of a kv head), partials in the split-K decode
 // layout (decode_scratch_floats(n_new * Hq, 128, num_splits) floats), then
-// split_rows_merge_launch.
+// their merge.
 hipError_t flash_prefill_keysplit_launch(uint16_t* out, const uint16_t* q, const uint8_t* k,
                                          const uint8_t* v, const float* k_scale,
                                          const float* v_scale, float* partial, int num_splits,

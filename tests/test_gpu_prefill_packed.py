@@ -82,6 +82,31 @@ def test_few_token_key_runs_match_oracle(n, clen, hq, hkv, splits):
     assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
 
 
+# The merge of the runs: a whole wave per row up to 4096 rows, half a wave
+# beyond, each in batches of 16 / 8 runs and maxima over 32: one run, two, the
+# edges of a batch and of the maximum's first load, and rows past one pass.
+@pytest.mark.parametrize("n,hq,hkv,tiles,run_tiles", [
+    (42, 24, 8, 2, 2), (42, 24, 8, 4, 2), (42, 24, 8, 32, 2), (42, 24, 8, 34, 2),
+    (42, 24, 8, 64, 2), (42, 24, 8, 66, 2), (64, 64, 8, 34, 2), (65, 64, 8, 8, 4),
+    (65, 64, 8, 32, 4), (65, 64, 8, 36, 4), (300, 64, 8, 17, 8)])
+def test_key_run_merge_matches_oracle(n, hq, hkv, tiles, run_tiles):
+    d, total = 128, 64 * tiles - 3
+    clen, splits = total - n, max(32, tiles // run_tiles)
+    q = O.normal_bf16((n, hq, d), 7600 + tiles)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7601 + tiles), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7602 + tiles), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    part.fill_(float("nan"))   # slots without a live run hold anything
+    step(f"merge n={n} hq={hq} tiles={tiles} splits={splits}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    want = O.attention_f32(q, k8, v8, ks, vs, n, clen, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(bf16_host(out), want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+
+
 def test_few_token_key_runs_refuse_what_the_decode_route_refused():
     hq, hkv, d = 17, 1, 128   # a group the MFMA decode kernel does not serve
     out = torch.empty((64, hq, d), dtype=torch.bfloat16, device=DEV)
