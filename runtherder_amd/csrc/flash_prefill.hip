@@ -177,13 +177,19 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
 
 // One LDS-DMA of 16 (or 4) bytes per lane: lane l's bytes land at LDS address
 // to + 16 l (4 l). In assembly, because the compiler waits for every
-// outstanding LDS-DMA before any LDS read; the waits here are explicit.
+// outstanding LDS-DMA before any LDS read; the waits here are explicit. The
+// base can come from a v_readfirstlane, and a vector-memory read of a scalar
+// register needs five wait states after a VALU write of it, which the hardware
+// does not check and the compiler does not count inside an asm. The s_mov_b64
+// makes the scalar ALU the last to write it (scalar reads and writes are
+// ordered by the hardware), and is the one wait state between the write of m0
+// and the copy.
 __device__ __forceinline__ void dma16(uint32_t to, const uint8_t* base, uint32_t off) {
     base = uniform_ptr(base);
     to   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(to)));
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(to), "v"(off), "s"(base)
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %0\n\tglobal_load_lds_dwordx4 %2, %0"
+                 : "+s"(base)
+                 : "s"(to), "v"(off)
                  : "memory");
 }
 // Lanes 0 .. kLanes - 1 only (the wave's lanes are all active).
