@@ -62,6 +62,7 @@
 
 #include "device_common.hpp"
 #include "launch.hpp"
+#include "prefill_tile.hpp"
 
 namespace rth {
 namespace {
@@ -70,7 +71,6 @@ typedef int      i32x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kBN     = 64;          // keys per tile
 constexpr int kHD     = 128;         // head_dim
 constexpr int kKTile  = kBN * kHD;   // bytes of E4M3 K codes per tile
 constexpr int kVPitch = kBN + 8;     // f16 per V^T row in LDS (144 B)
@@ -92,38 +92,6 @@ __device__ __forceinline__ int64_t packed_row(int r, int pack, int hq, int vhead
     const int t = r / pack;
     return static_cast<int64_t>(t) * hq + vhead * pack + (r - t * pack);
 }
-
-// Where a tile's rows are: key0 (clamped to the last tile, so that a copy past
-// the end repeats it), the last row that exists, and, paged, the offsets
-// (physical - logical key) of its two 32-key halves, each of which lies in
-// one block (blocks hold a power of two >= 32 keys).
-template <bool kPaged>
-struct TileRows {
-    int key0, rem, d_lo, d_hi;
-    __device__ __forceinline__ TileRows(int key0_, int total, const int* __restrict__ bt,
-                                        int bshift)
-        : key0(min(key0_, (total - 1) & ~(kBN - 1))), d_lo(0), d_hi(0) {
-        rem = total - 1 - key0;
-        if constexpr (kPaged) {
-            d_lo = (bt[key0 >> bshift] << bshift) - (key0 & ~((1 << bshift) - 1));
-            d_hi = d_lo;
-            if (rem >= 32) {
-                const int k1 = key0 + 32;
-                d_hi         = (bt[k1 >> bshift] << bshift) - (k1 & ~((1 << bshift) - 1));
-            }
-        }
-    }
-    // Byte offset of the tile's row 0 as half `hi` counts its rows. Signed when
-    // paged: the second half's block can lie at physical row 0, so that its
-    // row 0 counted from the tile's start is row -32.
-    __device__ __forceinline__ int64_t base(bool hi, uint32_t stride) const {
-        if constexpr (kPaged) {
-            return static_cast<int64_t>(key0 + (hi ? d_hi : d_lo)) * static_cast<int64_t>(stride);
-        } else {
-            return static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(key0)) * stride);
-        }
-    }
-};
 
 // Byte offset of 16-byte chunk c (0..7) of K row r (0..63) in an LDS K tile.
 __device__ __forceinline__ int k_chunk(int r, int c) {
@@ -211,7 +179,7 @@ template <int kWaves, bool kPaged>
 __device__ __forceinline__ void k_tile_dma(uint32_t dst, const uint8_t* __restrict__ kh,
                                            const TileRows<kPaged>& rows,
                                            const TileLane<kWaves>& ln, int wave) {
-    const uint32_t lim = static_cast<uint32_t>(rows.rem) * ln.kstride;
+    const uint32_t lim = rows.last_row(ln.kstride);
 #pragma unroll
     for (int rep = 0; rep < 8 / kWaves; ++rep) {
         const bool hi = kWaves == 8 ? wave >= 4 : rep == 1;
@@ -226,7 +194,7 @@ template <int kWaves, bool kPaged>
 __device__ __forceinline__ void v_tile_dma(uint32_t dst, const uint8_t* __restrict__ vh,
                                            const TileRows<kPaged>& rows,
                                            const TileLane<kWaves>& ln, int wave) {
-    const uint32_t lim  = static_cast<uint32_t>(rows.rem) * ln.kstride;
+    const uint32_t lim  = rows.last_row(ln.kstride);
     const uint8_t* base = vh + rows.base(wave >= kWaves / 2, ln.kstride);
     const uint32_t to   = dst + static_cast<uint32_t>(wave * (kKTile / kWaves));
     dma16(to, base, min(ln.vrow, lim) + ln.vcol);
@@ -242,7 +210,7 @@ __device__ __forceinline__ void scale_dma(uint32_t dst, const float* __restrict_
                                           const TileRows<kPaged>& rows,
                                           const TileLane<kWaves>& ln, int wave, int lane) {
     constexpr int  kKeys = 64 / kWaves;
-    const uint32_t lim   = static_cast<uint32_t>(rows.rem) * ln.sstride;
+    const uint32_t lim   = rows.last_row(ln.sstride);
     const int64_t  at    = rows.base(wave >= kWaves / 2, ln.sstride) + min(ln.srow, lim);
     const uint8_t* base  = reinterpret_cast<const uint8_t*>(lane < kKeys ? vsh : ksh);
     dma4_low<2 * kKeys>(dst + static_cast<uint32_t>(wave * 8 * kKeys), base + at);
