@@ -933,7 +933,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
         const int64_t row    = packed_row(row_e, pack, hq, vhead);
         const int64_t rows   = static_cast<int64_t>(n_new) * hq;
         const int64_t slot   = row * num_splits + static_cast<int64_t>(blockIdx.y);
-        const bool    any    = l_tot > 0.0f;
+        const bool    any    = !(l_tot == 0.0f);   // (a NaN row is one with keys)
         float*        part_o = partial + 2 * rows * num_splits + slot * kHD;
         if (he == 0) {
             partial[slot]                     = any ? m_ref : -INFINITY;

@@ -107,6 +107,59 @@ def test_key_run_merge_matches_oracle(n, hq, hkv, tiles, run_tiles):
     assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
 
 
+# A key whose score is NaN (an E4M3 NaN code, a NaN scale) or infinite (an
+# infinite scale) makes NaN of the rows that see it, in whichever of the runs it
+# lies, and of nothing else. (A row whose score is -inf keeps its other keys,
+# here and in the plain prefill; the oracle, which scales the codes first, makes
+# NaN of 0 x inf.)
+@pytest.mark.parametrize("what", ["k code", "k_scale nan", "k_scale inf", "v code"])
+@pytest.mark.parametrize("n,clen,splits,key", [
+    (48, 2000, 16, 5), (48, 2000, 16, 1000), (64, 3000, 16, 3030), (100, 3000, 16, 1500),
+    (250, 5000, 8, 5100)])
+def test_key_runs_propagate_nan(n, clen, splits, key, what):
+    hq, hkv, d, total = 32, 8, 128, clen + n
+    q = O.normal_bf16((n, hq, d), 7700 + n)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7701 + n), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7702 + n), d)
+    at = key * hkv + 3   # kv head 3
+    if what == "k code":
+        k8[at, 17] = 0x7F
+    elif what == "v code":
+        v8[at, 17] = 0x7F
+    else:
+        ks[at] = np.nan if what == "k_scale nan" else np.inf
+    out = torch.full((n, hq, d), 7.0, dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    step(f"key runs with a NaN: {what} n={n} clen={clen} splits={splits} key={key}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    got = O.bf16_to_f32(bf16_host(out))
+    plain = torch.full_like(out, 7.0)
+    R.flash_prefill_bf16(plain, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs), n,
+                         int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    plain = O.bf16_to_f32(bf16_host(plain))
+    with np.errstate(invalid="ignore"):
+        want = O.bf16_to_f32(O.attention_f32(q, k8, v8, ks, vs, n, clen, hq, hkv, d, d ** -0.5,
+                                             NTHREADS))
+    nan = np.isnan(want)
+    assert nan.any() and not nan.all()
+    if what == "v code":
+        # P V runs in MFMAs over 32 keys: a row of the key's tile that does not
+        # see it gets 0 x NaN, as in the plain prefill; rows after it all do.
+        first = max(0, key - clen)
+        assert np.isnan(got[first:, 12:16, 17]).all()
+        assert not np.isnan(np.delete(got, 17, axis=2)).any()
+        return
+    assert np.array_equal(np.isnan(got), np.isnan(plain))
+    if what == "k_scale inf":
+        assert np.isnan(got).any() and not np.isnan(got)[~nan].any()
+    else:
+        assert np.array_equal(np.isnan(got), nan)
+    assert np.abs(got - want)[~nan].max() <= 2e-2
+
+
 def test_few_token_key_runs_refuse_what_the_decode_route_refused():
     hq, hkv, d = 17, 1, 128   # a group the MFMA decode kernel does not serve
     out = torch.empty((64, hq, d), dtype=torch.bfloat16, device=DEV)
