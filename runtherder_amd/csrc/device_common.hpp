@@ -16,6 +16,9 @@ typedef float    f32x4 __attribute__((ext_vector_type(4)));
 typedef float    f32x16 __attribute__((ext_vector_type(16)));
 typedef float    f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// Four floats of the split scratch's O rows: these lie behind [rows, S] m and
+// [rows, S] l, 8-byte aligned where rows and S are odd.
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int   kWave     = 64;

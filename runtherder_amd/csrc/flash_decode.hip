@@ -1275,7 +1275,7 @@ __device__ __forceinline__ void decode_body(
             const int64_t row  = kMulti ? mrow(kvh0 + el, h) : (kvh0 + el) * G + h;
             const int64_t slot = row * num_splits + si;
             if (!kMulti || row >= 0) {
-                *reinterpret_cast<f32x4*>(&part_o[slot * D + d0]) = a;
+                *reinterpret_cast<f32x4_a4*>(&part_o[slot * D + d0]) = a;
             }
         }
         if (tid < pt.gkv * G) {
@@ -1315,7 +1315,7 @@ __device__ __forceinline__ void decode_body(
             for (int r = 0; r < 4; ++r) {
 #pragma unroll
                 for (int c = 0; c < T::kOMfma; c += 4) {
-                    *reinterpret_cast<f32x4*>(po + T::kVBytes * (4 * g + r) + c) =
+                    *reinterpret_cast<f32x4_a4*>(po + T::kVBytes * (4 * g + r) + c) =
                         f32x4{oacc[c][r], oacc[c + 1][r], oacc[c + 2][r], oacc[c + 3][r]};
                 }
             }
@@ -1502,7 +1502,8 @@ __global__ __launch_bounds__(kCombineThreads) void flash_decode_combine_kernel(
             const int s = min(s0 + u * kGroups, cap);
             ms[u]       = part_m[s];
             ls[u]       = part_l[s];
-            os[u]       = *reinterpret_cast<const f32x4*>(&part_o[static_cast<int64_t>(s) * D + 4 * qd]);
+            os[u] = *reinterpret_cast<const f32x4_a4*>(
+                &part_o[static_cast<int64_t>(s) * D + 4 * qd]);
         }
     };
     load8(grp, num_splits - 1);
@@ -1824,7 +1825,7 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_valu_kernel(
                 float*        o    = part_o + slot * D + 16 * j;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    *reinterpret_cast<f32x4*>(o + 4 * e) =
+                    *reinterpret_cast<f32x4_a4*>(o + 4 * e) =
                         f32x4{acc[h][4 * e], acc[h][4 * e + 1], acc[h][4 * e + 2], acc[h][4 * e + 3]};
                 }
                 if (j == 0) {

@@ -943,7 +943,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
         for (int db = 0; db < 4; ++db) {
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg) {
-                *reinterpret_cast<f32x4*>(part_o + 32 * db + 8 * rg + 4 * he) =
+                *reinterpret_cast<f32x4_a4*>(part_o + 32 * db + 8 * rg + 4 * he) =
                     any ? f32x4{o[db][4 * rg], o[db][4 * rg + 1], o[db][4 * rg + 2],
                                 o[db][4 * rg + 3]}
                         : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(kMergeThreads) void flash_prefill_merge_kernel(
                 const int i = min(s0 + u * kSub, live - 1);
                 m[u]        = pm[i];
                 ls[u]       = pl[i];
-                os[u]       = *reinterpret_cast<const f32x4*>(po + static_cast<int64_t>(i) * kHD);
+                os[u]       = *reinterpret_cast<const f32x4_a4*>(po + static_cast<int64_t>(i) * kHD);
             }
         };
         float big = pm[min(hl, live - 1)];   // M

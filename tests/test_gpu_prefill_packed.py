@@ -160,6 +160,56 @@ def test_key_runs_propagate_nan(n, clen, splits, key, what):
     assert np.abs(got - want)[~nan].max() <= 2e-2
 
 
+# An odd row count and an odd split count: the scratch's O rows start 8 bytes
+# past a 16-byte boundary. 81 tokens: key runs; 9: the decode kernel's route.
+@pytest.mark.parametrize("n", [81, 9])
+def test_odd_rows_and_splits_match_oracle(n):
+    hq, hkv, d, clen, splits = 7, 1, 128, 1000, 3
+    total = clen + n
+    q = O.normal_bf16((n, hq, d), 7800 + n)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7801 + n), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7802 + n), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    assert part.data_ptr() % 16 == 0 and n * hq * splits % 2 == 1
+    step(f"odd rows and splits n={n}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    want = O.attention_f32(q, k8, v8, ks, vs, n, clen, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(bf16_host(out), want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
+
+
+# Slabs and tensors that start 4 or 8 bytes past a 16-byte boundary (a view into
+# a larger buffer): the copies and stores are 16 bytes wide.
+@pytest.mark.parametrize("at", [4, 8])
+@pytest.mark.parametrize("n,clen", [(70, 100), (300, 60)])
+def test_slabs_off_a_16_byte_boundary(n, clen, at):
+    hq, hkv, d, total = 24, 8, 128, clen + n
+
+    def shifted(t):
+        raw = torch.zeros(t.numel() * t.element_size() + 16, dtype=torch.uint8, device=DEV)
+        got = raw[at:at + t.numel() * t.element_size()].view(t.dtype).view(t.shape)
+        got.copy_(t)
+        assert got.data_ptr() % 16 == at
+        return got
+
+    q = O.normal_bf16((n, hq, d), 7900 + n)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7901 + n), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7902 + n), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    got = shifted(out)
+    step(f"slabs {at} bytes off n={n} clen={clen}")
+    args = (n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    kv = (u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs))
+    R.flash_prefill_bf16(out, bf16_dev(q), *kv, *args)
+    R.flash_prefill_bf16(got, shifted(bf16_dev(q)), *map(shifted, kv), *args)
+    sync()
+    assert np.array_equal(bf16_host(got), bf16_host(out))
+    assert not torch.isnan(got).any()
+
+
 def test_few_token_key_runs_refuse_what_the_decode_route_refused():
     hq, hkv, d = 17, 1, 128   # a group the MFMA decode kernel does not serve
     out = torch.empty((64, hq, d), dtype=torch.bfloat16, device=DEV)
