@@ -997,21 +997,24 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void flash_prefill_kernel(
 // the count) -> with this one: empty cache 10.3 / 15.1 / 18.7 -> 9.0 / 11.1 /
 // 12.4 us, 1K keys 17.6 / 26.0 / 30.0 -> 13.6 / 22.9 / 26.0, 8K keys 26.5 /
 // 40.5 / 53.8 -> 23.5 / 41.0 / 51.6.
-// xcd_heads > 0 (kv heads a multiple of 8: the run kernel keeps a kv head on
-// one XCD, xcd_heads q heads on each): a workgroup (on XCD blockIdx.x % 8)
-// merges rows of its own XCD's heads, whose partials that XCD's L2 holds. Rows
-// in order reach the right XCD only where a workgroup's four rows are one kv
-// head's (groups of 4); the others read every partial across XCDs, 41-80 tokens
-// slower than the decode route at 300-2K keys. Per call, 64 tokens after 700 /
-// 1K / 2K keys, rows in order -> by XCD (decode route): 24 heads 15.6 / 16.4 /
-// 18.6 -> 14.3 / 14.1 / 15.6 us (14.9 / 16.0 / 18.4), 64 heads 21.1 / 24.1 /
-// 28.8 -> 17.4 / 20.0 / 23.7 (19.5 / 20.9 / 25.8), 32 heads 14.1 / 14.1 / 15.8
-// -> 14.2 / 14.2 / 15.8.
+// ways > 1: the run kernel's workgroups of a kv head lie on one XCD (kv heads a
+// multiple of 8: way_heads q heads on each) or on the 8 / ways XCDs x with x %
+// ways = the kv head (1, 2 or 4 kv heads): a merge workgroup (on XCD blockIdx.x
+// % 8) merges rows of its own XCD's heads, whose partials that XCD's L2 holds
+// (of 4 kv heads half, of 2 a quarter). Rows in order reach the right XCD only
+// where a workgroup's four rows are one kv head's (groups of 4); the others read
+// every partial across XCDs, 41-80 tokens slower than the decode route at
+// 300-2K keys. Per call, 64 tokens after 700 / 1K / 2K keys, rows in order ->
+// by XCD (decode route): 24 heads 15.6 / 16.4 / 18.6 -> 14.3 / 14.1 / 15.6 us
+// (14.9 / 16.0 / 18.4), 64 heads 21.1 / 24.1 / 28.8 -> 17.4 / 20.0 / 23.7 (19.5 /
+// 20.9 / 25.8), 32 heads 14.1 / 14.1 / 15.8 -> 14.2 / 14.2 / 15.8; 28 heads on 4
+// kv heads 15.1 / 15.9 / 18.1 -> 14.3 / 14.5 / 16.1 (14.8 / 16.3 / 18.5), at 41
+// tokens 14.3 / 14.8 / 16.9 -> 13.6 / 13.6 / 15.0 (14.2 / 14.2 / 16.3).
 constexpr int kMergeThreads = 256;
 template <int kSub>
 __global__ __launch_bounds__(kMergeThreads) void flash_prefill_merge_kernel(
     uint16_t* __restrict__ out, const float* __restrict__ partial, int num_splits,
-    const int* __restrict__ cache_len, int rows, int n_new, int run_min, int xcd_heads) {
+    const int* __restrict__ cache_len, int rows, int n_new, int run_min, int ways, int way_heads) {
     constexpr int kRows = kMergeThreads / (32 * kSub);
     static_assert(kSub == 1 || kSub == 2, "a row's lanes lie in one wave");
     const int tiles = (*cache_len + n_new + kBN - 1) / kBN;
@@ -1023,14 +1026,13 @@ __global__ __launch_bounds__(kMergeThreads) void flash_prefill_merge_kernel(
     const int     hl  = static_cast<int>(threadIdx.x) & 31;
     const int     sub = static_cast<int>(threadIdx.x) / 32 % kSub;
     const int64_t hs  = static_cast<int64_t>(rows) * num_splits;
-    // The rows of this workgroup's XCD (or all): row j of them is head j %
-    // xcd_heads of the XCD's heads, token j / xcd_heads.
-    const bool by_xcd = xcd_heads > 0;
-    const int  ways   = by_xcd ? 8 : 1;
-    const int  bid    = static_cast<int>(blockIdx.x);
+    // The rows of this workgroup's way (its XCD's, or all): row j of them is head
+    // j % way_heads of the way's heads, token j / way_heads.
+    const int bid = static_cast<int>(blockIdx.x);
     for (int j = bid / ways * kRows + static_cast<int>(threadIdx.x) / (32 * kSub);
          j < rows / ways; j += static_cast<int>(gridDim.x) / ways * kRows) {
-        const int row = by_xcd ? (j / xcd_heads * 8 + (bid & 7)) * xcd_heads + j % xcd_heads : j;
+        const int row =
+            ways > 1 ? (j / way_heads * ways + bid % ways) * way_heads + j % way_heads : j;
         const int64_t slot0 = static_cast<int64_t>(row) * num_splits;
         const float*  pm    = partial + slot0;
         const float*  pl    = partial + hs + slot0;
@@ -1144,11 +1146,11 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
     // 47.2 -> 40.6 / 47.9, 32K 100.4 / 123.8 -> 101.6 / 126.3.
     const bool wide = rows <= 4096;
     const int wgs = std::min((rows * (wide ? 64 : 32) + kMergeThreads - 1) / kMergeThreads, 2048);
+    const int ways = hkv % 8 == 0 ? 8 : 8 % hkv == 0 ? hkv : 1;
     // (A multiple of 8 workgroups: as many on each XCD.)
     hipLaunchKernelGGL(wide ? flash_prefill_merge_kernel<2> : flash_prefill_merge_kernel<1>,
                        dim3(static_cast<unsigned>((wgs + 7) & ~7)), dim3(kMergeThreads), 0, stream,
-                       out, partial, num_splits, cache_len, rows, n_new, run_min,
-                       hkv % 8 == 0 ? hq / 8 : 0);
+                       out, partial, num_splits, cache_len, rows, n_new, run_min, ways, hq / ways);
     return hipGetLastError();
 }
 

@@ -89,10 +89,11 @@ def test_few_token_key_runs_match_oracle(n, clen, hq, hkv, splits):
     (42, 24, 8, 2, 2), (42, 24, 8, 4, 2), (42, 24, 8, 32, 2), (42, 24, 8, 34, 2),
     (42, 24, 8, 64, 2), (42, 24, 8, 66, 2), (64, 64, 8, 34, 2), (65, 64, 8, 8, 4),
     (65, 64, 8, 32, 4), (65, 64, 8, 36, 4), (300, 64, 8, 17, 8),
-    # (rows by XCD: one and two kv heads each, groups of 1, 2 and 3; in order: 4
-    # and 5 kv heads)
+    # (rows by XCD: one and two kv heads each, groups of 1, 2 and 3; 4, 2 and 1 kv
+    # heads over two, four and all XCDs; in order: 5 and 12 kv heads)
     (81, 16, 16, 12, 4), (83, 48, 16, 9, 4), (99, 16, 8, 12, 4), (137, 48, 16, 17, 8),
-    (81, 28, 4, 12, 4), (101, 15, 5, 9, 4)])
+    (81, 28, 4, 12, 4), (45, 28, 4, 30, 2), (83, 10, 2, 9, 4), (201, 64, 2, 17, 8),
+    (97, 7, 1, 12, 4), (101, 15, 5, 9, 4), (82, 24, 12, 9, 4)])
 def test_key_run_merge_matches_oracle(n, hq, hkv, tiles, run_tiles):
     d, total = 128, 64 * tiles - 3
     clen, splits = total - n, max(32, tiles // run_tiles)
