@@ -1123,10 +1123,18 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
                                const int* block_table, int block_shift) {
     // A run's minimum of tiles, so that short caches use few runs: what another
     // run saves (1.05 us a tile) against the partials it writes for its rows
-    // and the merge reads (1K keys, 32 heads, minimum 2 / 4 / 8, us: 64 tokens
-    // 17.6 / 17.6 / 20.9; 128 tokens 26.1 / 22.6 / 25.1; 250 tokens 30.8 /
-    // 32.2 / 29.9).
-    const int     run_min = n_new <= 64 ? 2 : n_new <= 128 ? 4 : 8;
+    // and the merge reads, by the tokens up to 64 and from 81 on, by the rows
+    // between (where the runs took the decode route's place: that is the figure
+    // in brackets). After 300 / 1K / 2K keys, minimum 2 / 4 / 8, us: 64 tokens x 32
+    // heads 13.1 / 14.7 / 14.3, 13.7 / 15.1 / 19.0, 15.2 / 16.0 / 19.5; 80 x 24 heads
+    // 13.2 / 15.0 / 14.3 [14.1], 14.0 / 15.5 / 19.4 [17.5], 15.5 / 16.4 / 19.8 [21.6];
+    // 80 x 32 heads (2560 rows) 13.9 / 15.3 / 14.3 [14.7], 14.7 / 15.9 / 19.6 [18.2],
+    // 17.6 / 16.8 / 20.3 [22.3]; 80 x 64 heads 14.4 / 15.7 / 14.3 [19.3], 20.7 / 17.0 /
+    // 20.3 [25.6], 23.9 / 24.9 / 21.2 [35.4]; 128 x 32 heads 15.5 / 16.9 / 15.6, 20.4 /
+    // 17.8 / 21.2, 23.0 / 21.8 / 22.2; 200 x 32 heads 16.1 / 17.4 / 17.1, 21.8 / 20.3 /
+    // 21.4, 26.3 / 26.0 / 22.6.
+    const bool short_runs = n_new <= 64 || (n_new <= 80 && n_new * hq <= 2560);
+    const int  run_min    = short_runs ? 2 : n_new <= 128 ? 4 : 8;
     constexpr int kBM     = 32 * 4;
     const int     group = hq / hkv;
     const int     n_blk = (n_new * group + kBM - 1) / kBM;

@@ -60,12 +60,14 @@ def test_one_round_block_order(rounds, step_blocks):
 
 
 # Key runs of few tokens (41..80 with splits that fill the chip): run minimum
-# of 2 / 4 tiles on both sides of one run, ragged last runs, runs without keys
-# for the first rows, G = 3, 4, 7, and the split count just below the switch.
+# of 2 tiles and of 4 (from 65 tokens, over 2560 rows) on both sides of one run,
+# ragged last runs, runs without keys for the first rows, G = 3, 4, 6, 7, and the
+# split count just below the switch.
 @pytest.mark.parametrize("n,clen,hq,hkv,splits", [
     (41, 0, 24, 8, 32), (48, 80, 32, 8, 16), (48, 81, 32, 8, 16), (64, 64, 32, 8, 16),
     (64, 65, 32, 8, 16), (65, 191, 32, 8, 16), (66, 191, 32, 8, 16), (80, 1000, 28, 4, 22),
-    (80, 3001, 24, 8, 15), (50, 5000, 28, 4, 64), (64, 3000, 32, 8, 15)])
+    (80, 3001, 24, 8, 15), (50, 5000, 28, 4, 64), (64, 3000, 32, 8, 15),
+    (80, 48, 32, 8, 16), (80, 49, 32, 8, 16), (65, 191, 48, 8, 8), (66, 191, 48, 8, 8)])
 def test_few_token_key_runs_match_oracle(n, clen, hq, hkv, splits):
     d, total = 128, clen + n
     q = O.normal_bf16((n, hq, d), 7500 + n)
