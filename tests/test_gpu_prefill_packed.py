@@ -36,8 +36,13 @@ def run(n, clen, hq, hkv, seed):
     want = O.attention_f32(q[:first], k8, v8, ks, vs, first, clen, hq, hkv, d, d ** -0.5, NTHREADS)
     mx, mean = O.bf16_err(got[:first], want)
     assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
-    assert not np.isnan(got.astype(np.uint32) << 16).any()
-    return got
+    assert np.isfinite(O.bf16_to_f32(got)).all()
+    # Two tokens of every 128, the first and one inside.
+    for t in [t for b in range(40, n - 48, 128) for t in (b, min(b + 77, n - 1))]:
+        row = O.attention_f32(q[t:t + 1], k8, v8, ks, vs, 1, clen + t, hq, hkv, d, d ** -0.5,
+                              NTHREADS)
+        mx, mean = O.bf16_err(got[t:t + 1], row)
+        assert mx <= 2e-2 and mean <= 2e-3, (t, mx, mean)
 
 
 # (tokens, cached, q heads, kv heads): G = 7, 3, 5, 1, 32
@@ -50,7 +55,8 @@ def test_packed_rows_match_oracle(n, clen, hq, hkv):
 
 
 # Grids just below and above one 128-row workgroup per compute unit, and at the
-# end of the one-round ordering (two per compute unit): 8 kv heads, G = 1.
+# end of the one-round ordering (two per compute unit): 8 kv heads, G = 1. Every
+# row block is checked (run), the ones on both sides of the reordering among them.
 @pytest.mark.parametrize("step_blocks", [-1, 0, 1])
 @pytest.mark.parametrize("rounds", [1, 2])
 def test_one_round_block_order(rounds, step_blocks):
@@ -215,6 +221,25 @@ def test_slabs_off_a_16_byte_boundary(n, clen, at):
     sync()
     assert np.array_equal(bf16_host(got), bf16_host(out))
     assert not torch.isnan(got).any()
+
+
+# The most splits an entry takes, at few rows: most runs hold no key.
+@pytest.mark.parametrize("n", [41, 81])
+def test_most_splits(n):
+    hq, hkv, d, clen, splits = 1, 1, 128, 1000, 65536
+    total = clen + n
+    q = O.normal_bf16((n, hq, d), 7950 + n)
+    k8, ks = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7951 + n), d)
+    v8, vs = O.quantize_kv_fp8(O.normal_bf16((total * hkv, d), 7952 + n), d)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    step(f"most splits n={n}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(clen), hq, hkv, d, d ** -0.5)
+    sync()
+    want = O.attention_f32(q, k8, v8, ks, vs, n, clen, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(bf16_host(out), want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
 
 
 def test_few_token_key_runs_refuse_what_the_decode_route_refused():
