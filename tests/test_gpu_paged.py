@@ -151,12 +151,14 @@ def test_paged_fused_append_decode_equals_contiguous(total, block, hq, hkv):
     assert_attention_matches_oracle(got, qh, gk, gv, gks, gvs, 1, total - 1, hq, hkv, d)
 
 
-# Workgroup shapes on 256 compute units: 1021 and 3000 @ 2237 take the
-# key-split kernel, 200 (two 128-row blocks per head, whole grid resident) the
-# 4-wave kernel with heavy/light pairing, 2500 the 4-wave kernel over two
-# rounds (early-issue prologue), 4096 the 8-wave kernel.
+# Routes on 256 compute units: 1021 and 3000 @ 2237 take the 4-wave kernel in one
+# round, 2500 over two and a half, 4096 the 8-wave kernel; 200 tokens the key runs
+# (one run on the empty cache), and so do 48 and 80 (runs of two tiles or more), 100
+# (four) and 256 (eight).
 @pytest.mark.parametrize("total,clen,block", [(1021, 0, 64), (3000, 2237, 32), (4096, 0, 128),
-                                              (200, 0, 32), (1300, 1100, 64), (2500, 0, 64)])
+                                              (200, 0, 32), (1300, 1100, 64), (2500, 0, 64),
+                                              (3048, 3000, 64), (777, 697, 32), (1100, 1000, 32),
+                                              (2500, 2244, 128)])
 def test_paged_prefill_equals_contiguous(total, clen, block):
     hq, hkv, d = 32, 8, 128
     cont, paged, bt, table, _, _ = make_pair(total, hq, hkv, d, block, 50 + total)

@@ -87,9 +87,9 @@ def test_q_rows_of_extreme_magnitude(n):
     """q heads scaled from zero and bf16 subnormals up to 2^6 (scores several
     hundred apart between tiles). Tiny rows must keep a finite q split (their
     weights are near uniform); huge rows overflow P and rebase, and the other
-    rows of their wave must not be rebased downwards. n 300 runs the 4-wave
-    workgroup and n 700 the key-split one with the full oracle, n 4100 the
-    8-wave one on sampled rows."""
+    rows of their wave must not be rebased downwards. n 300 and 700 run the
+    4-wave workgroups with the full oracle, n 4100 the 8-wave ones on sampled
+    rows."""
     hq, hkv, d = (8, 2, 128) if n < 1000 else (32, 8, 128)
     scale = np.float32(1.0 / np.sqrt(d))
     f = np.tile(Q_FACTORS, hq // 8)
@@ -128,8 +128,8 @@ def test_q_rows_mixing_max_and_tiny_elements(n):
     """Every row mixes its maximum with elements down to 2^-22 of it: the
     scores come from the exact hi part, the lo part (large elements) and the
     subnormal-limited lo part (tiny elements); the output must still match
-    the oracle's scores, which use the bf16 q as is. n 300 / 700 / 4100 run
-    the 4-wave, key-split and 8-wave workgroups (the last on sampled rows)."""
+    the oracle's scores, which use the bf16 q as is. n 300 and 700 run the
+    4-wave workgroups, n 4100 the 8-wave ones (on sampled rows)."""
     hq, hkv, d = (8, 2, 128) if n < 1000 else (32, 8, 128)
     scale = np.float32(1.0 / np.sqrt(d))
     q = mixed_magnitude_q(n, hq, d, 44)
@@ -148,12 +148,10 @@ def test_q_rows_mixing_max_and_tiny_elements(n):
 @pytest.mark.parametrize("n_new,clen,hq,hkv", [
     (513, 0, 8, 2), (513, 129, 16, 4), (640, 64, 8, 8), (777, 1, 24, 8), (1500, 0, 8, 1),
 ])
-def test_key_split_workgroups(n_new, clen, hq, hkv):
-    """Grids of at most 1.5 rounds of 128-row blocks (4 or more per head)
-    split each block's key tiles over two halves of one workgroup (even and
-    odd tiles) and merge their (O, max, sum) at the end. Odd and even tile
-    counts, a cache prefix (the odd half's first tile fully masked for the
-    block's first rows when clen = 1), GQA groups of 1 to 8."""
+def test_mid_size_grids(n_new, clen, hq, hkv):
+    """4-wave grids of under one workgroup per compute unit, 10 to 94 row
+    blocks of 128: odd and even tile counts, a cache prefix, a last block of
+    one token, GQA groups of 1 to 8."""
     d = 128
     scale = np.float32(1.0 / np.sqrt(d))
     q, k8, v8, ks, vs = ref_inputs(n_new, clen, hq, hkv, d)
@@ -163,34 +161,28 @@ def test_key_split_workgroups(n_new, clen, hq, hkv):
     assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
 
 
-def shape_boundaries(cus, hq):
-    """Row counts at the edges of flash_prefill_launch's workgroup-shape choice
-    on a device with `cus` compute units (the same formulas as the launcher):
-    the last 4-wave / first key-split count (4 blocks of 128 rows), the last
-    key-split / first 4-wave count (2 * blocks * hq <= 3 * cus), and the first
-    8-wave count (ceil(n / 256) * hq >= 2 * cus)."""
-    out = [384, 385]
-    nb = (3 * cus) // (2 * hq)            # most 128-row blocks on the key split
-    if nb >= 4:
-        out += [128 * nb, 128 * nb + 1]
-    n8 = 256 * (-(-2 * cus // hq) - 1)     # last row count below the 8-wave path
-    out += [n8, n8 + 1]
-    return out
+def shape_boundaries(cus, hq, hkv):
+    """Token counts on both sides of flash_prefill_launch's choices on a device
+    with `cus` compute units (the same formulas as the launcher): one q head per
+    block / packed heads (64 tokens), at most one / more than one 4-wave workgroup
+    (128 rows) per compute unit, at most two / more (heavy and light blocks paired
+    or not), 4-wave / 8-wave (5 * ceil(rows / 256) * hkv >= 8 * cus)."""
+    group = hq // hkv
+    one   = cus // hkv * 128 // group
+    two   = 2 * cus // hkv * 128 // group
+    n8    = 256 * (-(-8 * cus // (5 * hkv)) - 1) // group   # the last 4-wave count
+    return [64, 65, one, one + 1, two, two + 1, n8, n8 + 1]
 
 
-@pytest.mark.parametrize("edge", range(6))
+@pytest.mark.parametrize("edge", range(8))
 def test_workgroup_shape_boundaries(edge):
-    """32 q heads at the edges of the launch's shape choice, derived from the
-    device's compute-unit count (on 256 CUs: 384 / 385 rows = 3 / 4 blocks of
-    128, 4-wave / key split; 1536 / 1537 = 12 / 13 blocks, key split / 4-wave;
-    3840 / 3841 = 15 / 16 blocks of 256, 4-wave / 8-wave). Sampled rows of
-    every block edge against the oracle."""
+    """32 q heads / 8 kv heads at the edges of the launch's choices, derived from
+    the device's compute-unit count (on 256 CUs: 64 / 65, 1024 / 1025, 2048 / 2049
+    and 3264 / 3265 tokens). Sampled rows of every block edge against the
+    oracle."""
     hq, hkv, d, clen = 32, 8, 128, 0
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    edges_n = shape_boundaries(cus, hq)
-    if edge >= len(edges_n):
-        pytest.skip(f"{cus} compute units leave no key-split range for {hq} heads")
-    n_new = edges_n[edge]
+    n_new = shape_boundaries(cus, hq, hkv)[edge]
     scale = np.float32(1.0 / np.sqrt(d))
     q, k8, v8, ks, vs = ref_inputs(n_new, clen, hq, hkv, d)
     got = gpu_prefill(q, k8, v8, ks, vs, n_new, clen, hq, hkv, d, scale)
@@ -296,9 +288,9 @@ def test_config4_prefill_sampled_rows(n):
 
 @pytest.mark.parametrize("clen", [0, 37, 100, 165])
 def test_large_grid_ragged_tile_counts(clen):
-    """n_new 4100 takes the 8-wave (two-group) path; with these cache lengths
-    the row blocks' tile counts cover every residue mod 4 of the unrolled tile
-    loop and the last tile is partial. Oracle on sampled rows."""
+    """n_new 4100 takes the 8-wave path; with these cache lengths the row blocks'
+    tile counts cover every residue mod 4 (the scales' ring; K's is three, V's
+    two) and the last tile is partial. Oracle on sampled rows."""
     hq, hkv, d, n = 32, 8, 128, 4100
     total = clen + n
     scale = np.float32(1.0 / np.sqrt(d))
@@ -420,12 +412,9 @@ def test_value_magnitudes_within_f16_staging(mag):
 
 
 def test_workgroup_shapes_agree_with_each_other():
-    """The three prefill workgroup shapes on the same heads: the key-split
-    kernel sums each row's exponentials as f16 p (v_dot2c, its register
-    budget), the 4- and 8-wave kernels as fp32 e; the P V MFMAs of all three
-    use f16 p. The heads are replicated so that one call takes each shape
-    (hq 8: key split, hq 128: 4-wave, hq 256: 8-wave); outputs of the same
-    head must agree within 2 bf16 ulps where |O| > 1e-2 and within 2e-4
+    """The 4-wave workgroups in one round, over several rounds and the 8-wave ones
+    on the same heads, replicated so that one call takes each (hq 8, 128, 256);
+    outputs of the same head must agree within 2 bf16 ulps where |O| > 1e-2 and within 2e-4
     elsewhere, and each with the oracle."""
     n, hq0, hkv0, d = 700, 8, 2, 128
     scale = np.float32(1.0 / np.sqrt(d))

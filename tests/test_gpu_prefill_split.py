@@ -145,11 +145,13 @@ def test_prefill_split_rejects_bad_arguments():
                                    k, s, s, part, 4, 2, int_dev(0), hq, hkv, 32, 0.1)
 
 
-@pytest.mark.parametrize("n_new", [2, 80, 81, 256, 257])
+@pytest.mark.parametrize("n_new", [2, 40, 41, 80, 81, 256, 257])
 def test_adaptive_backend_routes_small_prefill(n_new):
-    """AdaptiveAttention.run: 2..80 tokens take the split-K decode route over
-    the backend's scratch, 81..256 the flash prefill over key runs, 257 the
-    flash prefill; all match the oracle."""
+    """AdaptiveAttention.run: 2..40 tokens take the split-K decode route over
+    the backend's scratch, 41..256 the flash prefill over key runs, 257 the
+    flash prefill; all match the oracle. Which one ran shows in the scratch: on
+    an empty cache the key runs are one run, which stores the output itself and
+    leaves the scratch alone, the decode route writes its partials there."""
     hq, hkv, d, clen = 32, 8, 128, 3000
     scale = np.float32(1.0 / np.sqrt(d))
     q, k8, v8, ks, vs = inputs(n_new, clen, hq, hkv, d, 500 + n_new)
@@ -163,6 +165,15 @@ def test_adaptive_backend_routes_small_prefill(n_new):
     want = O.attention_f32(q, k8, v8, ks, vs, n_new, clen, hq, hkv, d, scale, NTHREADS)
     mx, mean = O.bf16_err(bf16_host(out), want)
     assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
+    runs = 40 < n_new <= 256
+    if runs:   # after the cache they do go through the scratch, and fill the chip
+        splits = be._split_prefill_splits(n_new)
+        assert splits * ((n_new * hq // hkv + 127) // 128) * hkv >= be.cus
+    be.partial.fill_(12345.0)
+    step(f"adaptive run n_new={n_new} on an empty cache")
+    be.run(out, bf16_dev(q), kv, n_new, int_dev(0))
+    sync()
+    assert bool((be.partial == 12345.0).all()) == (runs or n_new == 257)
 
 
 def test_adaptive_backend_small_prefill_paged_equals_contiguous():
