@@ -163,13 +163,14 @@ int rth_attn_prefill(uint16_t* out, const uint16_t* q, const uint8_t* k,
  * streaming every key (reference flash_prefill.cu:34-241 walks all keys
  * serially per tile: n_new = 4 at 32K keys costs ~50x a decode step).
  * n_new <= 80 (at head_dim 128 with splits that give the key runs a
- * workgroup per compute unit: <= 40), or head_dim != 128: the decode split kernel over (block of
- * tokens, kv head) units, token t over the first *cache_len + t + 1 keys
- * (shapes of the MFMA decode kernel, rth_decode_path == RTH_DECODE_MFMA:
- * head_dim 64 / 128 / 256; n_new <= 256). Beyond, at head_dim 128: the
- * flash prefill with each block of 128 rows (tokens x q heads of a kv head)
- * split over num_splits runs of key tiles. Both end in the decode merge. n_new's K/V must already be in the
- * cache (as for rth_attn_prefill). partial: rth_split_scratch_floats(n_new *
+ * workgroup per compute unit: <= 40), or head_dim != 128: the decode split
+ * kernel over (block of tokens, kv head) units, token t over the first
+ * *cache_len + t + 1 keys (shapes of the MFMA decode kernel, rth_decode_path
+ * == RTH_DECODE_MFMA: head_dim 64 / 128 / 256; n_new <= 256), and the decode's
+ * merge. Beyond, at head_dim 128: the flash prefill with each block of 128
+ * rows (tokens x q heads of a kv head) split over num_splits runs of key
+ * tiles, and a merge of their own. n_new's K/V must already be in the cache
+ * (as for rth_attn_prefill). partial: rth_split_scratch_floats(n_new *
  * num_q_heads, head_dim, num_splits) floats, no initialization needed;
  * 1 <= n_new <= 4096. Results match rth_attn_prefill within the attention
  * tolerance (a different summation order). */

@@ -8,8 +8,9 @@
 // tokens after a long cache as split-K decode; 16 tokens after 8K keys 209 ->
 // 17 us per call, at an empty cache up to ~2 us slower), and at head_dim 128
 // calls of up to kPrefillRunsTokens tokens run it as the flash prefill over
-// key runs (64 / 128 / 250 tokens after 32K keys 897 / 828 / 829 -> 51 / 83 /
-// 149 us; at an empty cache 2-6 us slower). For those the scratch holds
+// key runs (64 / 128 / 250 tokens after 32K keys, the flash prefill -> the runs,
+// 517 / 533 / 538 -> 56 / 88 / 157 us; at an empty cache 2 us slower). For those
+// the scratch holds
 // kPrefillRunTokenRuns token-runs (34 MB at 32 q heads).
 #pragma once
 

@@ -38,9 +38,10 @@ inline void flash_prefill_bf16(__hip_bfloat16*       out,
 }
 
 // No reference counterpart: the same attention split over the keys
-// (rth_attn_prefill_split): up to 80 tokens as split-K decode over (token
-// block, kv head) units, beyond as the flash prefill over num_splits key runs
-// per (row block, q head); partial holds flash_split_scratch_floats(n_new *
+// (rth_attn_prefill_split): up to 80 tokens (40 at head_dim 128 with splits
+// that fill the chip) as split-K decode over (token block, kv head) units,
+// beyond as the flash prefill over num_splits key runs per block of 128 rows
+// (tokens x q heads of a kv head); partial holds flash_split_scratch_floats(n_new *
 // num_q_heads, head_dim, num_splits) floats.
 inline void flash_prefill_split_bf16(__hip_bfloat16*       out,
                                      const __hip_bfloat16* q,

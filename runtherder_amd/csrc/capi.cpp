@@ -155,12 +155,20 @@ int prefill_split_common(uint16_t* out, const uint16_t* q, const uint8_t* k, con
     // block, kv head) units; beyond, the flash prefill over key runs. That
     // also from kPrefillSplitRunTokens + 1 tokens where num_splits gives it a
     // workgroup per compute unit: every block of tokens of the decode route
-    // reads the whole cache again (32 heads, decode route / 16 runs, us: 64
-    // tokens after 32K keys 86.6 / 51.1, 8K 31.0 / 26.5, 1K 15.6 / 17.6, none
-    // 9.5 / 11.0; 48 tokens 85.8 / 48.0, 30.4 / 25.6, 15.5 / 16.3, 9.0 / 10.7;
-    // 32 tokens 50.8 / 42, 22.0 / 23.6, 13.2 / 14.6, 7.9 / 10.1). With the few
-    // splits that suit the decode route (num_splits around CUs / n_new) it
-    // stays there.
+    // reads the whole cache again. With the few splits that suit the decode
+    // route (num_splits around CUs / n_new) it stays there. Decode route / key
+    // runs with the backend's splits, after none / 300 / 1K / 4K / 16K keys, us:
+    //   64 tokens x 32 heads 9.2 / 8.6, 13.5 / 13.0, 15.5 / 13.5, 22.2 / 17.6, 48.9 / 32.3
+    //   41 x 32 heads 8.7 / 8.7, 13.7 / 12.4, 16.1 / 13.0, 27.2 / 16.7, 79.1 / 31.1
+    //   41 x 24 heads 8.0 / 8.7, 11.8 / 12.3, 13.3 / 12.6, 18.3 / 15.6, 36.2 / 24.6
+    //   41 x 28 heads on 4: 8.4 / 8.7, 10.5 / 13.1, 14.2 / 13.6, 19.6 / 17.7, 44.7 / 27.1
+    //   41 x 16 heads on 2: 7.7 / 8.5, 9.7 / 12.4, 13.6 / 13.2, 16.8 / 17.1, 30.8 / 23.0
+    // Below the line the same holds from 17 tokens on: the runs are the faster
+    // ones from 1K keys up (but for 32 tokens x 32 heads after 4K, 17.7 / 19.3),
+    // the decode route up to 300 (17 x 32 heads 7.5 / 8.2, 8.9 / 10.9, 13.0 / 11.3,
+    // 18.3 / 13.8; 40 x 32 heads 8.2 / 8.7, 12.2 / 12.4, 13.9 / 13.1, 18.8 / 16.0). The
+    // depth is not known here; the few tokens stay on the route that costs a
+    // short cache least.
     bool runs = head_dim == 128 && n_new > rth::kPrefillSplitDecodeTokens;
     if (head_dim == 128 && !runs && n_new > rth::kPrefillSplitRunTokens &&
         rth::decode_mfma_supported(num_q_heads, num_kv_heads, head_dim)) {

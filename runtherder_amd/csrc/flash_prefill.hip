@@ -44,14 +44,17 @@
 //    MFMAs ahead. Before, a wave did scores, softmax and P V one after the
 //    other, and the compiler put a wait for all outstanding copies in front of
 //    each tile's reads. What bounds it: one wave per SIMD (4-wave grids of up
-//    to one workgroup per compute unit) issues ~340 instructions per tile at
-//    one per ~5 cycles, 1.05 us a tile (1.6 before); two waves per SIMD run at
-//    57 % of the MFMA rate at ~1.9 GHz, where the part's power holds it (a
-//    large bf16 matrix product: 1.23 PFLOP/s; this kernel at 16384 tokens, 32
-//    heads 1.15). Measured, before -> now, us: 24 heads 1021 / 1500 / 1800
-//    tokens 27.2 -> 24.5, 34.8 -> 33.3, 43.3 -> 38.9; 28 heads 1700 48.4 ->
-//    37.5; 32 heads 2048 / 3000 / 4096 / 16384 55.4 -> 47.1, 97 -> 85.6, 139
-//    -> 136, 1913 -> 1905.
+//    to one workgroup per compute unit) takes ~2410 cycles a tile, 1.02 us at
+//    2.36 GHz (1.6 us before): ~340 instructions, 1024 cycles of MFMAs and the
+//    softmax and staging, which one wave overlaps in part only; two waves per
+//    SIMD run at 57 % of the MFMA rate at ~1.9 GHz, where the part's power
+//    holds it (a large bf16 matrix product: 1.23 PFLOP/s; this kernel at 16384
+//    tokens, 32 heads 1.13-1.16). Measured, before -> now, us, both built and
+//    timed in turn: 24 heads 1021 / 1700 / 3000 tokens 26.9 -> 23.3, 40.0 -> 35.7,
+//    86.4 -> 69.2; 28 heads 1700 47.9 -> 36.4; 32 heads 1021 / 2048 / 3000 / 4096
+//    27.0 -> 23.5, 55.3 -> 45.6, 95.8 -> 84.2, 142 -> 136. At the power limit it
+//    is even: 32 heads 8192 / 16384 517 -> 508 (runs differ by 7 %), 1960 -> 1949,
+//    4096 after 64K / 127K keys 3894 -> 3905, 7406 -> 7432, there 0.3-0.5 % slower.
 //  * Key runs (flash_prefill_keysplit_launch, kPart): for chunks after a long
 //    cache, each row block of the 4-wave kernel is split over gridDim.y
 //    workgroups, each walking one run of key tiles and storing partials in the
@@ -1122,7 +1125,7 @@ hipError_t launch_prefill_part(uint16_t* out, const uint16_t* q, const uint8_t* 
                                int hq, int hkv, float scale_log2, hipStream_t stream,
                                const int* block_table, int block_shift) {
     // A run's minimum of tiles, so that short caches use few runs: what another
-    // run saves (1.05 us a tile) against the partials it writes for its rows
+    // run saves (1.02 us a tile) against the partials it writes for its rows
     // and the merge reads, by the tokens up to 64 and from 81 on, by the rows
     // between (where the runs took the decode route's place: that is the figure
     // in brackets). After 300 / 1K / 2K keys, minimum 2 / 4 / 8, us: 64 tokens x 32

@@ -197,9 +197,9 @@ def flash_prefill_split_bf16(out, q, k, v, k_scale, v_scale, partial, num_splits
     (no reference counterpart; the reference walks every key serially per q
     tile, flash_prefill.cu:34-241): up to 80 tokens (40, where num_splits
     fills the chip at head_dim 128) as split-K decode over (token block, kv
-    head) units, beyond (head_dim 128) the flash prefill over num_splits key
-    runs per block of 128 rows, both merged by the decode
-    merge. partial: flash_split_scratch_floats(n_new * num_q_heads, head_dim,
+    head) units with the decode's merge, beyond (head_dim 128) the flash prefill
+    over num_splits key runs per block of 128 rows with a merge of their own.
+    partial: flash_split_scratch_floats(n_new * num_q_heads, head_dim,
     num_splits) floats; 1 <= n_new <= PREFILL_SPLIT_MAX_TOKENS."""
     _need(out, torch.bfloat16, "out"); _need(q, torch.bfloat16, "q")
     _need(k, torch.uint8, "k"); _need(v, torch.uint8, "v")
@@ -459,9 +459,9 @@ class AdaptiveAttention(AttentionBackend):
     (2 n_new) splits (no reference counterpart: per call, 16 tokens after 8K
     keys 209 -> 17 us; at an empty cache up to ~2 us slower); at head_dim 128,
     calls of up to PREFILL_RUNS_TOKENS tokens take it as the flash prefill
-    over key runs (64 / 128 / 250 tokens after 32K keys 897 / 828 / 829 -> 51
-    / 83 / 149 us; at an empty cache 2-6 us slower), for which the scratch
-    holds PREFILL_RUN_TOKEN_RUNS token-runs."""
+    over key runs (64 / 128 / 250 tokens after 32K keys, the flash prefill ->
+    the runs, 517 / 533 / 538 -> 56 / 88 / 157 us; at an empty cache 2 us
+    slower), for which the scratch holds PREFILL_RUN_TOKEN_RUNS token-runs."""
 
     def __init__(self, config: AttnConfig, num_splits: int | None = None, device="cuda"):
         self.config = config
