@@ -12,6 +12,7 @@ import torch
 import oracle_lib as O
 import runtherder_amd as R
 from gpu_util import DEV, NTHREADS, bf16_dev, bf16_host, f32_dev, int_dev, step, sync, u8_dev
+from test_gpu_prefill import dynamic_range_inputs, mixed_magnitude_q
 
 pytestmark = pytest.mark.gpu
 
@@ -171,6 +172,28 @@ def test_key_runs_propagate_nan(n, clen, splits, key, what):
     else:
         assert np.array_equal(np.isnan(got), nan)
     assert np.abs(got - want)[~nan].max() <= 2e-2
+
+
+# Scores that jump by hundreds between the runs and q rows whose elements span 22
+# binades, through the key runs' own reference maxima and the merge.
+@pytest.mark.parametrize("what", ["score range", "mixed q"])
+@pytest.mark.parametrize("n,splits", [(48, 16), (100, 16), (250, 8)])
+def test_key_runs_dynamic_range(n, splits, what):
+    hq, hkv, d, total = 32, 8, 128, 1300
+    q, k8, v8, ks, vs = dynamic_range_inputs(total, hq, hkv, d)
+    q = q[-n:]
+    if what == "mixed q":
+        q = mixed_magnitude_q(n, hq, d, 46)
+        ks = np.minimum(ks, np.float32(0.02))   # (the score range alone is the other case)
+    out = torch.full((n, hq, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    part = R.new_flash_split_scratch(n * hq, d, splits)
+    step(f"key runs, {what} n={n} splits={splits}")
+    R.flash_prefill_split_bf16(out, bf16_dev(q), u8_dev(k8), u8_dev(v8), f32_dev(ks), f32_dev(vs),
+                               part, splits, n, int_dev(total - n), hq, hkv, d, d ** -0.5)
+    sync()
+    want = O.attention_f32(q, k8, v8, ks, vs, n, total - n, hq, hkv, d, d ** -0.5, NTHREADS)
+    mx, mean = O.bf16_err(bf16_host(out), want)
+    assert mx <= 2e-2 and mean <= 2e-3, (mx, mean)
 
 
 # An odd row count and an odd split count: the scratch's O rows start 8 bytes
