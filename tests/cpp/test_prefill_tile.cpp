@@ -17,11 +17,13 @@ long long checked = 0;
 // key min(key0 + r, total - 1) has.
 template <bool kPaged>
 bool check(int key0, int total, uint32_t stride, const int* bt, int shift) {
-    const rth::TileRows<kPaged> t(key0, total, bt, shift);
+    using Rows = rth::TileRows<kPaged>;
+    const Rows t(key0, total, Rows::entries(key0, total, bt, shift), shift);
     const int from = std::min(key0, (total - 1) / rth::kBN * rth::kBN);
     for (int r = 0; r < rth::kBN; ++r) {
-        const uint32_t off  = std::min(static_cast<uint32_t>(r) * stride, t.last_row(stride));
-        const int64_t  got  = t.base(r >= 32, stride) + off;
+        const bool     hi   = r >= 32;
+        const uint32_t off  = t.offset(hi, static_cast<uint32_t>(r & 31) * stride, stride);
+        const int64_t  got  = static_cast<int64_t>(t.base(hi, stride)) + off;
         const int64_t  key  = std::min<int64_t>(from + r, total - 1);
         const int64_t  row  = kPaged ? (static_cast<int64_t>(bt[key >> shift]) << shift) +
                                            (key & ((1 << shift) - 1))

@@ -1,12 +1,15 @@
-"""Wait states that the hardware does not check (CPU only: compiles the kernels
-to gfx950 assembly with the library's own flags). A vector-memory instruction
+"""What the kernels' gfx950 assembly must and must not hold (CPU only: compiled
+with the library's own flags). First the wait states that the hardware does not
+check: a vector-memory instruction
 may read a scalar register only five wait states or more after a vector ALU
 instruction wrote it (AMD's CDNA instruction set guides, manually inserted
 wait states). The compiler keeps that distance for its own instructions but
 does not look into inline assembly, where the prefill issues its LDS copies."""
+import functools
 import re
 import shutil
 import subprocess
+import tempfile
 from pathlib import Path
 
 import pytest
@@ -75,15 +78,47 @@ def test_the_check_sees_a_short_distance():
     assert short_distances(head + " s_nop 3\n" + load)[1] == 1
 
 
-@pytest.mark.skipif(shutil.which(B.HIPCC) is None and not Path(B.HIPCC).exists(),
-                    reason="hipcc not available")
-@pytest.mark.parametrize("src", ASM_SOURCES)
-def test_scalar_bases_of_memory_instructions_have_settled(src, tmp_path):
-    out = tmp_path / "k.s"
+@functools.lru_cache(maxsize=None)
+def assembly(src):
     flags = [f for f in B.DEVICE_FLAGS if f != "-fPIC"]
-    res = subprocess.run([B.HIPCC, *flags, "-x", "hip", "--cuda-device-only", "-S",
-                          str(B.CSRC / src), "-o", str(out)], capture_output=True, text=True)
-    assert res.returncode == 0, res.stderr[-2000:]
-    bad, seen = short_distances(out.read_text())
+    with tempfile.TemporaryDirectory() as d:
+        out = Path(d) / "k.s"
+        res = subprocess.run([B.HIPCC, *flags, "-x", "hip", "--cuda-device-only", "-S",
+                              str(B.CSRC / src), "-o", str(out)], capture_output=True, text=True)
+        assert res.returncode == 0, res.stderr[-2000:]
+        return out.read_text()
+
+
+needs_hipcc = pytest.mark.skipif(shutil.which(B.HIPCC) is None and not Path(B.HIPCC).exists(),
+                                 reason="hipcc not available")
+
+
+@needs_hipcc
+@pytest.mark.parametrize("src", ASM_SOURCES)
+def test_scalar_bases_of_memory_instructions_have_settled(src):
+    bad, seen = short_distances(assembly(src))
     assert seen > 50, f"only {seen} memory instructions with a scalar base parsed"
     assert not bad, f"{len(bad)} of {seen}: " + "; ".join(bad[:4])
+
+
+@needs_hipcc
+def test_prefill_tile_loop_waits_for_no_scalar_load():
+    """The prefill's tile loop (it holds the third barrier of each kernel) has no
+    scalar load, whose round trip every tile would wait for, and takes values out
+    of vector registers only for a paged cache's two block-table entries."""
+    text, seen = assembly("flash_prefill.hip"), 0
+    for m in re.finditer(r"^(_Z\w*flash_prefill_kernelILi\dELb(\d)\w*):.*?^\.Lfunc_end", text,
+                         re.M | re.S):
+        code = [line.split(";")[0].strip() for line in m[0].splitlines()]
+        at = [i for i, line in enumerate(code) if line == "s_barrier"][2]
+        # From the loop's head (the target of the first branch back past the barrier).
+        label = {line[:-1]: i for i, line in enumerate(code) if re.match(r"\.LBB\w+:", line)}
+        end, head = next((i, label[t[1]]) for i, line in enumerate(code[at:], at)
+                         if (t := re.match(r"s_c?branch\w* (\.LBB\w+)", line)) and label[t[1]] < at)
+        loop = code[head:end]
+        assert sum("mfma" in line for line in loop) == 24, m[1]
+        assert not [line for line in loop if line.startswith("s_load")], m[1]
+        taken = sum(line.startswith("v_readfirstlane") for line in loop)
+        assert taken == (2 if m[2] == "1" else 0), (m[1], taken)
+        seen += 1
+    assert seen == 6
