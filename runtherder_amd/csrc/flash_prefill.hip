@@ -47,14 +47,13 @@
 //    to one workgroup per compute unit) takes ~2410 cycles a tile, 1.02 us at
 //    2.36 GHz (1.6 us before): ~340 instructions, 1024 cycles of MFMAs and the
 //    softmax and staging, which one wave overlaps in part only; two waves per
-//    SIMD run at 57 % of the MFMA rate at ~1.9 GHz, where the part's power
+//    SIMD run at 60 % of the MFMA rate at ~1.9 GHz, where the part's power
 //    holds it (a large bf16 matrix product: 1.23 PFLOP/s; this kernel at 16384
-//    tokens, 32 heads 1.13-1.16). Measured, before -> now, us, both built and
-//    timed in turn: 24 heads 1021 / 1700 / 3000 tokens 26.9 -> 23.3, 40.0 -> 35.7,
-//    86.4 -> 69.2; 28 heads 1700 47.9 -> 36.4; 32 heads 1021 / 2048 / 3000 / 4096
-//    27.0 -> 23.5, 55.3 -> 45.6, 95.8 -> 84.2, 142 -> 136. At the power limit it
-//    is even: 32 heads 8192 / 16384 517 -> 508 (runs differ by 7 %), 1960 -> 1949,
-//    4096 after 64K / 127K keys 3894 -> 3905, 7406 -> 7432, there 0.3-0.5 % slower.
+//    tokens, 32 heads 1.15-1.18). Measured, before -> now, us, both built and
+//    timed in turn: 24 heads 1021 / 1700 / 3000 tokens 27.0 -> 23.4, 39.6 -> 35.4,
+//    86.3 -> 69.2; 28 heads 1700 48.0 -> 36.8; 32 heads 1021 / 2048 / 3000 / 4096
+//    27.0 -> 23.4, 55.3 -> 45.3, 96.1 -> 84.4, 141 -> 133; 8192 / 16384 tokens 511 ->
+//    493, 1927 -> 1883, 4096 after 32K / 127K keys 1977 -> 1946, 7449 -> 7283.
 //  * Key runs (flash_prefill_keysplit_launch, kPart): for chunks after a long
 //    cache, each row block of the 4-wave kernel is split over gridDim.y
 //    workgroups, each walking one run of key tiles and storing partials in the
